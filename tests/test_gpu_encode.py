@@ -67,3 +67,57 @@ def test_encode_many_tiles_persistent(te, gpu_device):
     bits_g, _ = te.encode_tiles(torch.from_numpy(w).to(gpu_device), 3, "mcg", want_dq=False)
     bits_o, _, _ = ov.viterbi_tb(w, 3, tn.codebook_lut("mcg"))
     assert np.array_equal(bits_g.cpu().numpy().view(np.uint32), tn.pack_bits(bits_o, 3))
+
+
+def _encode_np(w, K, lut):
+    """The two-pass encode of one tile in numpy fp32, with q = 0 where no candidate lies below
+    FLT_MAX (the C oracle leaves such a step's backpointer as it was)."""
+    E, Q, top = 1 << (16 - K), 1 << K, np.float32(np.finfo(np.float32).max)
+    v = lut.reshape(Q, E)
+
+    def one(seq, overlap):
+        cost = np.zeros(E, np.float32)
+        if overlap is not None:
+            cost[:] = top / np.float32(4)
+            cost[overlap] = 0
+        back = []
+        for t in range(256):
+            d = np.float32(seq[t]) - v
+            c = d * d + np.repeat(cost.reshape(Q, E >> K), Q, axis=1)
+            c = np.where(c < top, c, top)            # also NaN -> FLT_MAX
+            q = c.argmin(0)                          # the smallest q on ties
+            cost = c[q, np.arange(E)]
+            back.append(q)
+        e = int(cost.argmin()) if overlap is None else overlap
+        states = np.empty(256, np.int64)
+        for t in range(255, -1, -1):
+            states[t] = (int(back[t][e]) << (16 - K)) | e
+            e = int(states[t]) >> K
+        return states
+
+    first = one(np.roll(w, 128), None)
+    return one(w, int(first[128]) >> K)
+
+
+@pytest.mark.parametrize("K", [2, 3, 4])
+@pytest.mark.parametrize("cb", ["mcg", "1mad"])
+def test_encode_ties_and_non_finite_targets(te, gpu_device, K, cb):
+    """Targets whose minimum is shared by many candidates (zeros, constants, magnitudes that
+    swamp the codebook), and ones whose costs overflow or are NaN, where no candidate lies
+    below FLT_MAX and q = 0 stands: the path equals the plain fp32 passes, bit for bit."""
+    _say(f"[encode] ties and non-finite K={K} cb={cb}")
+    rng = np.random.default_rng(K)
+    rows = [np.zeros(256), np.tile([1.0, -1.0], 128), np.full(256, 1e6), np.full(256, -3e18),
+            np.full(256, 1.5e19), np.full(256, np.inf), np.full(256, np.nan)]
+    for at, v in ((0, np.nan), (127, np.inf), (128, -np.inf), (255, np.nan), (200, 1.2e19)):
+        row = rng.standard_normal(256)
+        row[at] = v
+        rows.append(row)
+    w = np.stack(rows).astype(np.float32)
+    lut = tn.codebook_lut(cb)
+    with np.errstate(all="ignore"):
+        states = np.stack([_encode_np(r, K, lut) for r in w])
+    bits_g, dq_g = te.encode_tiles(torch.from_numpy(w).to(gpu_device), K, cb)
+    want = tn.pack_bits((states & ((1 << K) - 1)).astype(np.int32), K)
+    assert np.array_equal(bits_g.cpu().numpy().view(np.uint32), want)
+    assert np.array_equal(dq_g.cpu().numpy().view(np.uint32), lut[states].view(np.uint32))

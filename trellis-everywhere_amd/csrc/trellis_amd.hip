@@ -531,7 +531,7 @@ int trellis_embed_rows(const trellis_desc* W, const int32_t* tokens, int ntok, v
 int trellis_encode_workspace_bytes(int K, uint32_t ntiles, size_t* bytes) {
   if (!bytes) return TRELLIS_ERR_NULL;
   if (K < 2 || K > 4) return TRELLIS_ERR_K;
-  *bytes = static_cast<size_t>(encode_grid(ntiles)) * vit_bp_bytes(K);
+  *bytes = static_cast<size_t>(encode_grid(ntiles)) * VIT_BP_BYTES;
   return TRELLIS_OK;
 }
 
@@ -542,7 +542,7 @@ int trellis_encode_tiles(const float* w, uint32_t ntiles, int K, int codebook, u
   if (ntiles == 0) return TRELLIS_OK;
   if (!w || !bits) return TRELLIS_ERR_NULL;
   const unsigned grid = encode_grid(ntiles);
-  if (!workspace || ws_bytes < static_cast<size_t>(grid) * vit_bp_bytes(K))
+  if (!workspace || ws_bytes < static_cast<size_t>(grid) * VIT_BP_BYTES)
     return TRELLIS_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(workspace) % 256) return TRELLIS_ERR_ALIGN;
   VitArgs a;
