@@ -1,34 +1,27 @@
-// bgemm.h — batched packed linear for gfx950 (batch 2 .. prefill): decode once, reuse
-// across the batch.
+// bgemm.h — batched packed linear for gfx950: decode once, reuse across the batch. Three
+// kernels by the call's rows, each a 128-row output block (the out-dim Hadamard block) x a
+// block of batch columns x one k-range per workgroup, one workgroup per CU:
+//   bgemm16_kernel    up to 16 rows: 16 waves, activations shared through LDS;
+//   bgemm_kernel      32 or 64 columns: 8 waves, each with its own share of the k-range;
+//   bgemm_wide_kernel 128 or 256 columns: 4 waves with 64 accumulator tiles each.
+// In each a wave decodes a tile once, straight into the A operand of an MFMA (common.h), and
+// multiplies it with every column of the block. With one k-range the workgroup applies
+// y = sv * osc * Hb_n(t) itself, otherwise it stores its partial block and bfold_kernel (next
+// launch) adds the slices in slice order and folds, one wave per batch column: reducing
+// inside the kernel leaves the whole reduction to the last workgroup of each block, behind
+// device-scope round trips, and measured slower.
 //
-// A workgroup of 16 waves (12 for the exact mode's 128-column blocks) owns one 128-row
-// output block (the out-dim Hadamard block) x NB = 16*NC batch columns x one k-range of
-// `kr` tile columns, walked in steps of KT tiles (16 at 16 columns, 8 up to 64 and in the
-// fp16-weight mode, 6 for the exact mode's 128 columns). Wave w = (band group
-// bg = w % NG, k-lane kl = w / NG), a band group being BW = 2 or 4 adjacent bands
-// (NG = 8 / BW groups, KL = waves / NG k-lanes): the waves of a SIMD share a band group and
-// split every step's tiles between them (tile j of a step belongs to k-lane j % KL), so a
-// SIMD has four (or three) waves to switch between:
-//   * the B tile of a step (xf[batch cols][KT*16] as (x, x) fp16 pairs written by
-//     xfold_kernel) is loaded two steps ahead into registers by all the threads, stored
-//     to one half of a double-buffered LDS area, and read by every wave: each fragment
-//     serves the BW bands of each of the NG band groups; one barrier per step;
-//   * each wave's packed words ride a two-step register ring and a wave-private LDS
-//     buffer (for the lanes' window reads), as in gemv_kernel;
-//   * each wave decodes a tile of each of its bands once, straight into the A operand of
-//     v_mfma_f32_16x16x32_f16 (the exact (hi, lo) pair against the duplicated activation,
-//     common.h), and issues NC MFMAs per band against the NC batch chunks;
-//   * every load is a range-checked buffer load (batch rows past the call's, tiles past the
-//     matrix read zeros), so none is clamped or skipped and the waits stay exact;
-//   * the B rows are padded by 8 words (a row stride of 8 mod 64 words): the 16 batch
-//     rows x 4 column groups of a fragment read then run at the LDS's full rate on gfx950
-//     (measured 177 B/clk per CU, against 115 with a 4-word pad, whose rows collide);
-//   * the epilogue adds the KL k-lanes' sums into t[NB][128] in LDS in k-lane order
-//     (deterministic); with one k-range the workgroup applies y = sv * osc * Hb_n(t)
-//     itself, otherwise it stores its partial block and bfold_kernel (next launch) adds
-//     the slices in slice order and folds, one wave per batch column: reducing inside the
-//     kernel leaves the whole reduction to the last workgroup of each block, behind
-//     device-scope round trips, and measured slower.
+// Measured on the Qwen3-8B block (K=3, MCG, one MI355X, the two sides in turn on one box; the
+// one before is a 16-wave workgroup, 12 for exact 128-column blocks, whose waves shared B tiles
+// double-buffered in LDS with a barrier per step of 6 to 8 tile columns):
+//   gate+up, 32 / 64 / 128 rows, exact            32.6 / 42-44 / 68.2 -> 28.3 / 38.5 / 64.9 us
+//   gate+up, 512 rows, exact                      229-235 -> 205-208 us
+//   down, 2048 rows, exact / fp16-weight mode     438-445 / 280-289 -> 333-342 / 236-240 us
+// What bounds them: the GPU's power limit sets the clock once the matrix cores work on real
+// activations (gate+up at 512 rows ran at 1.56 GHz with 32x32x16 MFMAs, and at 2.33 GHz, 1.4
+// times as fast, with all-zero activations), then instruction issue (a wave issues at most
+// one operation per 5 cycles; decode, MFMA issue and LDS reads add up to ~1.3 times the
+// matrix time of an exact 128-column block).
 #pragma once
 
 #include "common.h"
@@ -90,44 +83,7 @@ __device__ __forceinline__ void bg_out_fold(const LinArgs& g, const LinMat& m, c
   }
 }
 
-// k-step: 16 tile columns for 16 batch columns (half the barriers; the 8B gate+up group at
-// batch 16: 29.1 -> 27.9 us), 8 for up to 64, 6 for 128 (two per k-lane over three
-// k-lanes; LDS holds two B steps; a k-range's last step may be partial); always 8 in the
-// fp16-weight mode, whose B words are half as many per column
-template <int NC, int F16> struct BgStep {
-  static constexpr int KT = F16 ? 8 : NC == 1 ? 16 : NC <= 4 ? 8 : 6;
-};
-// waves per workgroup: 16 (four per SIMD), or 12 (three per SIMD, up to 168 registers each)
-// for the exact mode's 128-column blocks, whose 8 fragments and 16 accumulators per wave
-// (~150 registers) do not fit a quarter of a SIMD's registers (against 8 waves, two per
-// SIMD: the 8B block at a 512 prefill 463.4 -> 452.2 us, gate+up at 128 rows 69.4 -> 64.9)
-template <int NC, int F16> struct BgWaves {
-  static constexpr int WV = (!F16 && NC == 8) ? 12 : 16;
-};
-// bands per wave: 4 at 16 batch columns (8 k-lanes: each B fragment read from LDS feeds 4
-// bands instead of 2; the 8B gate+up group at batch 16 27.8 -> 26.6-27.1 us), otherwise 2
-// (a band pair, 4 k-lanes: at 32 and 64 columns 4 bands measured no faster on gate+up and
-// 4-6 % slower on the split-K launches, whose epilogue adds twice the k-lanes); the k-step
-// must hold a tile column per k-lane
-template <int NC, int F16> struct BgBands {
-  static constexpr int BW = (!F16 && NC == 1) ? 4 : 2;
-};
-// LDS regions of the epilogue's t[NB][TLS] partial sums, one per k-lane added in the same
-// round (the k-lanes' sums meet in KL / NR rounds): as many as the LDS holds beside the
-// waves' packed-word buffers, up to one per k-lane. From 64 batch columns (one workgroup per
-// CU whatever its LDS) the whole LDS; below that half of it, so a kernel with few registers
-// keeps room for two workgroups per CU (the 8B gate+up group at batch 16, four regions
-// instead of two: 26.1 -> 25.9 us, 29.2 -> 28.7 in the fp16-weight mode).
 constexpr int BG_LDS_WORDS = 160 * 1024 / 4;
-template <int NC> __host__ __device__ constexpr int bg_regions(int nb, int kl, int tls, int xbuf,
-                                                              int other) {
-  // below 64 columns the LDS stays within half a CU's, for two workgroups per CU
-  const int limit = NC < 4 ? BG_LDS_WORDS / 2 : BG_LDS_WORDS;
-  const int base = 2 * xbuf;
-  int r = kl;
-  while (r > 1 && (r * nb * tls > base ? r * nb * tls : base) + other > limit) r /= 2;
-  return r;
-}
 
 // s_setprio with a value known after unrolling (the instruction takes an immediate)
 __device__ __forceinline__ void setprio_n(int v) {
@@ -137,12 +93,33 @@ __device__ __forceinline__ void setprio_n(int v) {
   else __builtin_amdgcn_s_setprio(0);
 }
 
-template <int K, int CB, int V, int NC, int F16, bool SINGLE>
-__global__ __launch_bounds__((64 * BgWaves<NC, F16>::WV)) void bgemm_kernel(LinArgs g) {
-  constexpr int BG_WAVES = BgWaves<NC, F16>::WV;
+// ---------------------------------------------------------------- up to 16 columns
+// A workgroup of 16 waves: wave w = (band group bg = w % NG, k-lane kl = w / NG), a band group
+// being BW adjacent bands; the waves of a SIMD share a band group and split every k-step's
+// tiles between them (tile j of a step belongs to k-lane j % KL):
+//   * the B tile of a step (xf[batch cols][KT*16] as (x, x) fp16 pairs written by
+//     xfold_kernel) is loaded two steps ahead into registers by all the threads, stored
+//     to one half of a double-buffered LDS area, and read by every wave: each fragment
+//     serves the BW bands of each of the NG band groups; one barrier per step;
+//   * each wave's packed words ride a two-step register ring and a wave-private LDS buffer
+//     (for the lanes' window reads);
+//   * every load is a range-checked buffer load (batch rows past the call's, tiles past the
+//     matrix read zeros), so none is clamped or skipped and the waits stay exact;
+//   * the B rows are padded by 8 words (a row stride of 8 mod 64 words: the fragments' reads
+//     spread over the banks);
+//   * the epilogue adds the k-lanes' sums into t[16][128] in LDS in k-lane order.
+// At 16 rows the kernels for more columns measured slower (8B gate+up 28.9 us with 32-column
+// blocks, 26.5 with this one; q/k/v 16.5 and 15.9, o 14.7 and 13.2, down 19.5 and 17.3).
+template <int K, int CB, int V, int F16, bool SINGLE>
+__global__ __launch_bounds__(1024) void bgemm16_kernel(LinArgs g) {
+  constexpr int NC = 1, BG_WAVES = 16;
   constexpr int NWK = 8 * K;
-  constexpr int KT = BgStep<NC, F16>::KT;          // tile columns per k-step
-  constexpr int BW = BgBands<NC, F16>::BW;         // bands per wave
+  // tile columns per k-step: 16 (half the barriers of 8; the 8B gate+up group 29.1 -> 27.9 us),
+  // 8 in the fp16-weight mode, a pair per k-lane
+  constexpr int KT = F16 ? 8 : 16;
+  // bands per wave: 4 (8 k-lanes; each B fragment read from LDS feeds 4 bands: 27.8 ->
+  // 26.6-27.1 us), 2 in the fp16-weight mode
+  constexpr int BW = F16 ? 2 : 4;
   constexpr int NG = 8 / BW;                       // band groups of the block
   constexpr int KL = BG_WAVES / NG;                // k-lanes: waves of one band group
   // tiles per band per k-lane per step: exact mode, tiles kl, kl + KL, ...; fp16-weight
@@ -151,7 +128,7 @@ __global__ __launch_bounds__((64 * BgWaves<NC, F16>::WV)) void bgemm_kernel(LinA
   static_assert(F16 || (KT % KL == 0 && TPL >= 1), "a tile column per k-lane per step");
   constexpr int WPT = F16 ? 8 : 16;                // B words per tile column and batch row
   constexpr int XW = KT * WPT + 8;                 // LDS words per B row (+8: bank spread)
-  constexpr int NB = 16 * NC;                      // batch columns per workgroup
+  constexpr int NB = 16;                           // batch columns per workgroup
   constexpr int RCH = KT * WPT / 4;                // 16-byte chunks per B row per step
   constexpr int XCH = NB * RCH;                    // 16-byte B chunks per step
   constexpr int XLOADS = (XCH + 64 * BG_WAVES - 1) / (64 * BG_WAVES);
@@ -161,14 +138,15 @@ __global__ __launch_bounds__((64 * BgWaves<NC, F16>::WV)) void bgemm_kernel(LinA
   constexpr int BLOADS = (BCH + 63) / 64;
   constexpr int BSW = BLOADS * 256;                // words per wave buffer: every lane's chunks
   static_assert(!F16 || (KT == 2 * KL && BW == 2), "fp16-weight mode: one tile pair per k-lane per step");
-  // epilogue: t[NB][TLS] (rows padded like the B rows, so a fragment's float4 writes
-  // spread over the banks) in NR regions NR_OFF floats apart over the B buffers (bg_regions:
-  // k-lanes k2 .. k2 + NR - 1 add into regions 0 .. NR - 1 in round k2 / NR)
+  // epilogue: t[NB][TLS] (rows padded like the B rows, so a fragment's float4 writes spread
+  // over the banks) in NR regions NR_OFF floats apart over the B buffers (k-lanes
+  // k2 .. k2 + NR - 1 add into regions 0 .. NR - 1 in round k2 / NR). Four regions: more
+  // would leave no room for two workgroups per CU (against two: 26.1 -> 25.9 us)
   constexpr int TLS = 136;
-  constexpr int NR = bg_regions<NC>(NB, KL, TLS, XBUF, BG_WAVES * BSW);
+  constexpr int NR = 4;
   constexpr int NR_OFF = NB * TLS;
   constexpr int XSB = 2 * XBUF > NR * NR_OFF ? 2 * XBUF : NR * NR_OFF;
-  static_assert(KL % NR == 0 && NB * TLS <= XSB, "epilogue regions");
+  static_assert(KL % NR == 0 && XSB + BG_WAVES * BSW <= BG_LDS_WORDS / 2, "epilogue regions");
   __shared__ __align__(16) uint32_t xsb[XSB];
   __shared__ __align__(16) uint32_t bst[BG_WAVES * BSW];
   float* tl = reinterpret_cast<float*>(xsb);
@@ -404,6 +382,579 @@ __global__ __launch_bounds__((64 * BgWaves<NC, F16>::WV)) void bgemm_kernel(LinA
     return;
   }
   bg_out_fold<CB, BG_WAVES, TLS, NR, NR_OFF, NB>(g, m, tl, ob, b0, nbv, rows, sov);
+}
+
+// The work item of a workgroup: workgroups go round the 8 XCDs, so the ones of an XCD (b % 8)
+// take a contiguous run of items, in order.
+__device__ __forceinline__ int xcd_item(int b, int total) {
+  constexpr int XCDS = 8;
+  const int q = total / XCDS, rem = total % XCDS, x = b % XCDS;
+  return x * q + min(x, rem) + b / XCDS;
+}
+
+// y = sv * osc * Hb_n(t) of the nbe columns t[c] (BG_TLS floats apart, summed over NR regions
+// NR_OFF floats apart) of batch rows b0 .. b0 + nbe - 1. Eight columns a wave at a time, eight
+// lanes a column, 16 rows a lane: the Hadamard's levels 1 to 8 are plain adds in the lane,
+// 16 to 64 butterflies over the 8 lanes (signs as in fwht_chunk, joined to the scale), the
+// sums read and the rows written 16 bytes at a time. About 35 instructions a column, against
+// ~70 with a column across the 64 lanes, which the waves of these kernels, one or two to a
+// SIMD, issue at 5 cycles each. so = sv * osc of the lane's rows.
+constexpr int BG_TLS = 132;    // floats per column of t (4 mod 64: a wave's writes spread over the banks)
+template <int CB, int WAVES, int NR, int NR_OFF, int EC>
+__device__ __forceinline__ void bg_fold16(const LinArgs& g, const LinMat& m, const float* tl, int ob,
+                                          int b0, int nbe, int rows, const float (&so)[16]) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int l8 = lane & 7;
+  const FwhtLane fl = fwht_lane(lane, 8);
+  const int B = m.block_out;                    // 16 to 128
+  // the sign a(l) that the butterflies leave in the lane
+  const int cross = B > 64 ? 7 : B > 32 ? 3 : B > 16 ? 1 : 0;
+  const float nrm = (__builtin_popcount(l8 & cross) & 1) ? -m.nrm_out : m.nrm_out;
+#pragma unroll
+  for (int c0 = 0; c0 < EC; c0 += 8 * WAVES) {
+    const int c = c0 + 8 * wave + (lane >> 3);
+    if (c0 + 8 * wave >= nbe) break;
+    const float4_t* t4 = reinterpret_cast<const float4_t*>(tl + c * BG_TLS + 16 * l8);
+    float v[16];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float4_t q = t4[j];
+#pragma unroll
+      for (int n = 1; n < NR; ++n) q += t4[n * (NR_OFF / 4) + j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[4 * j + i] = CB == CB_1MAD ? q[i] / 147.800537109375f : q[i];
+    }
+#pragma unroll
+    for (int d = 1; d < 16; d *= 2)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (!(i & d)) {
+          const float a = v[i], b = v[i + d];
+          v[i] = a + b;
+          v[i + d] = a - b;
+        }
+    if (B > 16)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) butterfly<1>(v[i], v[i + 1], fl.s1, lane);
+    if (B > 32)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) butterfly<2>(v[i], v[i + 1], fl.s2, lane);
+    if (B > 64)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) butterfly<4>(v[i], v[i + 1], fl.s4, lane);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] *= so[i] * nrm;
+    // rows of a band past the matrix and columns past the call's are not stored
+    const bool keep = c < nbe && 16 * l8 < rows;
+    const long long o = static_cast<long long>(b0 + c) * m.ldy + ob * 128 + 16 * l8;
+    if (g.y_f16) {
+      uint32_t h[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const half2_t p = {static_cast<_Float16>(v[2 * i]), static_cast<_Float16>(v[2 * i + 1])};
+        h[i] = __builtin_bit_cast(uint32_t, p);
+      }
+      _Float16* y = static_cast<_Float16*>(m.y) + o;
+      if (!keep) {
+      } else if (m.y_words) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) st_wt16(y + 8 * i, u32x4_t{h[4 * i], h[4 * i + 1], h[4 * i + 2], h[4 * i + 3]});
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st_wt(y + i, static_cast<_Float16>(v[i]));
+      }
+    } else if (keep) {
+      float* y = static_cast<float*>(m.y) + o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        st_wt16(y + 4 * i, __builtin_bit_cast(u32x4_t, float4_t{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]}));
+    }
+  }
+}
+
+// The epilogue of the kernels below: the KL k-lanes' sums meet in LDS as t[column][row], EC
+// columns at a time, in NR regions (one per k-lane, or the k-lanes in KL / NR rounds), added
+// in a fixed order; then the output fold, or with split-K the partial block for bfold_kernel.
+// put(region, e, add) writes (adds) the calling wave's sums of the e-th EC columns. The rounds
+// are separated by barriers that leave the stores in flight (lds_barrier).
+template <int CB, int NC, int WAVES, int KL, int NR, class Put>
+__device__ __forceinline__ void bg_epilogue(const LinArgs& g, const LinMat& m, uint32_t* lds, int kl,
+                                            int ob, int cb, int sl, int rows, Put put) {
+  constexpr int NB = 16 * NC, EC = NB < 64 ? NB : 64, NR_OFF = EC * BG_TLS;
+  float* tl = reinterpret_cast<float*>(lds);
+  const int b0 = cb * NB, ncb = (g.batch + NB - 1) / NB;
+  const int nbv = min(NB, g.batch - b0);
+  // one k-range: the output scales of the lane's rows (zeros past the matrix); they arrive
+  // while the sums meet
+  float4_t sv[4], os[4];
+  if (m.S == 1) {
+    const rsrc_t r_sv = make_rsrc(m.sv + ob * 128, rows * 4), r_os = make_rsrc(m.osc + ob * 128, rows * 4);
+    const int o = (threadIdx.x & 7) * 64;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sv[j] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r_sv, o + 16 * j, 0, 0));
+      os[j] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r_os, o + 16 * j, 0, 0));
+    }
+  }
+  lds_barrier();   // every wave is done with its ring: the sums take its place
+#pragma unroll
+  for (int e = 0; e < NB / EC; ++e) {
+    const int nbe = min(EC, nbv - e * EC);
+    if (nbe <= 0) break;
+    if (e > 0) lds_barrier();
+#pragma unroll
+    for (int k2 = 0; k2 < KL; k2 += NR) {
+      if (kl >= k2 && kl < k2 + NR) put(tl + (kl - k2) * NR_OFF, e, k2 > 0);
+      lds_barrier();
+    }
+    if (m.S > 1) {
+      // publish this slice's partial block (16-byte write-through stores)
+      float* mypart = m.part + (static_cast<size_t>(ob * ncb + cb) * m.S + sl) * NB * 128 + e * EC * 128;
+      const float4_t* t4 = reinterpret_cast<const float4_t*>(tl);
+      const rsrc_t r_p = make_rsrc(mypart, static_cast<unsigned>(nbe) * 512);
+      for (int i = threadIdx.x; i < nbe * 32; i += 64 * WAVES) {
+        const int j = (i >> 5) * (BG_TLS / 4) + (i & 31);
+        float4_t v = t4[j];
+#pragma unroll
+        for (int q = 1; q < NR; ++q) v += t4[q * (NR_OFF / 4) + j];
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r_p, i * 16, 0, AUX_SC1);
+      }
+    } else {
+      float so[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) so[i] = sv[i / 4][i % 4] * os[i / 4][i % 4];
+      bg_fold16<CB, WAVES, NR, NR_OFF, EC>(g, m, tl, ob, b0 + e * EC, nbe, rows, so);
+    }
+  }
+}
+
+// ---------------------------------------------------------------- 17 to 64 columns
+// One workgroup of 8 waves (two per SIMD, up to 256 registers each) per 128-row output block
+// x 32 CC batch columns x k-range, on v_mfma_f32_32x32x16_f16. A wave owns all four band
+// pairs x all the columns, and a contiguous share of the k-range, so every fragment of A and
+// B is used without another wave's help and nothing in the loop is shared: each wave streams
+// its packed words and its B fragments from global memory straight into LDS rings of its own
+// (load_lds16) and waits only for its own loads. No barrier, no staging registers, no LDS
+// store.
+template <int NC> struct BgShape {
+  static constexpr int CC = NC / 2;             // 32-column chunks
+  static constexpr int RG = 4;                  // band pairs per wave
+  static constexpr int WAVES = 8;
+  static constexpr int KL = 8;                  // the waves' shares of the k-range
+  static constexpr int T = 4;                   // tile columns per stage of packed words
+  static constexpr int PB = 4;                  // tile columns of B in flight (ring slots)
+};
+
+template <int K, int CB, int V, int NC, int F16, bool SINGLE>
+__global__ __launch_bounds__(512) void bgemm_kernel(LinArgs g) {
+  using Sh = BgShape<NC>;
+  constexpr int CC = Sh::CC, RG = Sh::RG, KL = Sh::KL, T = Sh::T, PB = Sh::PB, WAVES = Sh::WAVES;
+  constexpr int NB = 32 * CC;                   // batch columns per workgroup
+  constexpr int NWK = 8 * K, CPT = 2 * K;       // words, 16-byte chunks per tile
+  constexpr int BW = 2 * RG;                    // bands per wave
+  constexpr int BCH = BW * T * CPT;             // chunks of a wave's stage of packed words
+  constexpr int BL = (BCH + 63) / 64;           // load instructions for them
+  constexpr int BST = BL * 256;                 // words of a stage slot
+  constexpr int XST = CC * 256;                 // words of a B slot (one tile column)
+  constexpr int RING = 2 * BST + PB * XST;
+  // the exact mode: a weight's two halves side by side in one operand, against B's values
+  // duplicated in registers (4 v_perm_b32 per quad, shared by the wave's four band pairs)
+  constexpr bool SUM = F16 || CB == CB_1MAD;    // one fp16 per weight (1MAD: exactly)
+  constexpr int NR = CC == 1 ? KL : 4, EC = NB;   // epilogue regions, columns per round
+  constexpr int WORDS = WAVES * RING > NR * EC * BG_TLS ? WAVES * RING : NR * EC * BG_TLS;
+  static_assert(WORDS <= BG_LDS_WORDS && KL % NR == 0, "rings and epilogue regions fit the LDS");
+  static_assert(T == PB && T % 2 == 0, "static ring slots and read-ahead registers");
+  static_assert(PB <= T && PB * CC + BL + CC < 64, "loads in flight");
+  __shared__ __align__(16) uint32_t lds[WORDS];
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int item = xcd_item(blockIdx.x, g.total);
+  const int mi = SINGLE ? 0 : locate_mat(g, item, false);
+  const LinMat& m = g.m[mi];
+  {
+    // the matrix's fields that the set-up needs, loaded in one round
+    const int f_i0 = m.item0, f_s = m.S, f_t = m.tiles_in, f_n = m.n, f_ob = m.n_ob;
+    const int f_bt = g.batch, f_kr = g.kr;
+    const uint32_t *f_b = m.bits, *f_xf = m.xf;
+    const float *f_sv = m.sv, *f_os = m.osc;
+    asm volatile("" ::"s"(f_i0), "s"(f_s), "s"(f_t), "s"(f_n), "s"(f_ob), "s"(f_bt), "s"(f_kr),
+                 "s"(f_b), "s"(f_xf), "s"(f_sv), "s"(f_os));
+  }
+  // items: column blocks outermost, so that the workgroups in flight on an XCD read one
+  // block's activations, which its L2 then holds; then output blocks, then k-ranges
+  const int local = item - m.item0;
+  const int sl = local % m.S, cbob = local / m.S;
+  const int cb = cbob / m.n_ob, ob = cbob % m.n_ob;
+  const int rows = min(128, m.n - ob * 128);
+  const int kl = wave;                          // share of the k-range
+  const int ntl = min(g.kr, m.tiles_in - sl * g.kr);
+  const int share = (ntl + KL - 1) / KL;
+  const int j0 = sl * g.kr + kl * share;        // this wave's tile columns j0 .. j0 + nt - 1
+  const int nt = min(share, ntl - kl * share);  // (none: nt <= 0)
+
+  // ---- loads: per-lane offsets, fixed; the column's part is one add
+  const size_t blk0 = static_cast<size_t>(ob) * 8 * m.tiles_in * NWK;
+  const int nbands = min(8, m.n / 16 - ob * 8);  // bands of this block in the matrix
+  const rsrc_t r_b = make_rsrc(m.bits + blk0, static_cast<unsigned>(nbands * m.tiles_in * NWK * 4));
+  const int nch32 = (g.batch + XF_CHUNK - 1) / XF_CHUNK;
+  const rsrc_t r_x = make_rsrc(reinterpret_cast<const char*>(m.xf) +
+                                   static_cast<size_t>(cb) * CC * m.tiles_in * XF_FRAG,
+                               static_cast<unsigned>(min(CC, nch32 - cb * CC)) * m.tiles_in * XF_FRAG);
+  // packed words: chunk ch of a stage = band ch / (T CPT), then the band's T tiles in order
+  unsigned boff[BL], bt[BL];
+#pragma unroll
+  for (int q = 0; q < BL; ++q) {
+    const int ch = lane + 64 * q;
+    const int bb = ch / (T * CPT), rem = ch % (T * CPT);
+    bt[q] = rem / CPT;                          // tile of the stage
+    boff[q] = ch < BCH ? static_cast<unsigned>((bb * m.tiles_in + j0) * NWK * 4 + rem * 16)
+                       : RSRC_PAST;
+  }
+  uint32_t* ring = lds + wave * RING;
+  const unsigned ring_base = __builtin_amdgcn_readfirstlane(lds_addr(ring));
+  auto load_bits = [&](int s) {
+#pragma unroll
+    for (int q = 0; q < BL; ++q) {
+      // tiles past the wave's share are not read
+      const unsigned o = static_cast<int>(s * T + bt[q]) < nt ? boff[q] + static_cast<unsigned>(s * T * NWK * 4) : RSRC_PAST;
+      load_lds16<false>(r_b, ring_base + static_cast<unsigned>((s & 1) * BST * 4 + q * 1024), o);
+    }
+  };
+  const unsigned xcs = static_cast<unsigned>(m.tiles_in) * XF_FRAG;   // bytes per chunk
+  const unsigned xoff = static_cast<unsigned>(j0) * XF_FRAG + lane * 16;
+  auto load_x = [&](int c, int slot) {
+    const unsigned o = c < nt ? xoff + static_cast<unsigned>(c) * XF_FRAG : RSRC_PAST;
+#pragma unroll
+    for (int q = 0; q < CC; ++q)
+      load_lds16<false>(r_x, ring_base + static_cast<unsigned>((2 * BST + slot * XST) * 4 + q * 1024), o + q * xcs);
+  };
+
+  const int r = lane & 15, h = lane >> 5;
+  const QuadPos q0 = quad_pos_v<K, V>(r, h), q1 = quad_pos_v<K, V>(r, h + 2);
+  const uint32_t* wbase = ring + ((lane >> 4) & 1) * T * NWK;
+  const uint32_t* xbase = ring + 2 * BST + lane * 4;
+  float16_t acc[RG][CC];
+#pragma unroll
+  for (int p = 0; p < RG; ++p)
+#pragma unroll
+    for (int c = 0; c < CC; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[p][c][i] = 0.f;
+
+  // every load that the compiler knows of has landed: it puts no wait of its own after the
+  // ring's loads, which it cannot count
+  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+  asm volatile("" ::: "memory");
+
+  load_bits(0);
+#pragma unroll
+  for (int c = 0; c < PB; ++c) load_x(c, c);
+  // a column's fragments and window words, read from LDS one column ahead of their use
+  u32x4_t bx[2][CC];
+  uint32_t w[2][RG][4];
+  auto read_column = [&](const uint32_t* wst, int t, u32x4_t (&b)[CC], uint32_t (&v)[RG][4]) {
+#pragma unroll
+    for (int c = 0; c < CC; ++c)
+      b[c] = *reinterpret_cast<const u32x4_t*>(xbase + t * XST + c * 256);
+#pragma unroll
+    for (int p = 0; p < RG; ++p) {
+      const uint32_t* tp = wst + (2 * p * T + t) * NWK;
+      v[p][0] = tp[q0.wa];
+      v[p][1] = tp[q0.wb];
+      v[p][2] = tp[q1.wa];
+      v[p][3] = tp[q1.wb];
+    }
+  };
+  auto compute = [&](const u32x4_t (&b)[CC], const uint32_t (&v)[RG][4]) {
+    if constexpr (SUM) {
+#pragma unroll
+      for (int p = 0; p < RG; ++p) {
+        uint32_t p0[4], p1[4];
+        decode_lcg<K, CB, V>(v[p][0], v[p][1], q0.sh, p0);
+        decode_lcg<K, CB, V>(v[p][2], v[p][3], q1.sh, p1);
+        const half8_t A = operand_sum<CB>(p0, p1);
+#pragma unroll
+        for (int c = 0; c < CC; ++c)
+          acc[p][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, __builtin_bit_cast(half8_t, b[c]), acc[p][c], 0, 0, 0);
+      }
+    } else {
+      half8_t d0[CC], d1[CC];
+#pragma unroll
+      for (int c = 0; c < CC; ++c) {
+        d0[c] = dup_frag(b[c], 0);
+        d1[c] = dup_frag(b[c], 1);
+      }
+#pragma unroll
+      for (int p = 0; p < RG; ++p) {
+        uint32_t pv[4];
+        decode_lcg<K, CB, V>(v[p][0], v[p][1], q0.sh, pv);
+        const half8_t A0 = operand_pairs(pv);
+#pragma unroll
+        for (int c = 0; c < CC; ++c)
+          acc[p][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0, d0[c], acc[p][c], 0, 0, 0);
+        decode_lcg<K, CB, V>(v[p][2], v[p][3], q1.sh, pv);
+        const half8_t A1 = operand_pairs(pv);
+#pragma unroll
+        for (int c = 0; c < CC; ++c)
+          acc[p][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, d1[c], acc[p][c], 0, 0, 0);
+      }
+    }
+  };
+  // loads land in issue order: column 0's fragments (and stage 0's words before them) have
+  // landed when at most the other PB - 1 columns' are outstanding
+  wait_vmcnt<(PB - 1) * CC>();
+  asm volatile("" ::: "memory");
+  read_column(wbase, 0, bx[0], w[0]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const int nst = (nt + T - 1) / T;
+  for (int s = 0; s < nst; ++s) {
+    // a SIMD issues from its older wave first: each wave's priority falls as its share is
+    // done, so that the two finish together
+    setprio_n((4 * (nst - s) - 1) / nst);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      // the slots refilled here were read into registers in the column (the words: the stage)
+      // before, and those reads have returned
+      if (t == 0) load_bits(s + 1);
+      load_x(s * T + t + PB, t);
+      // after the next column's fragments (and its stage's words before them) came PB - 1
+      // columns of fragments and, up to column PB - 2, the next stage's words
+      if (t + 1 < PB)
+        wait_vmcnt<(PB - 1) * CC + BL>();
+      else
+        wait_vmcnt<(PB - 1) * CC>();
+      asm volatile("" ::: "memory");
+      read_column(wbase + ((t + 1 < T ? s : s + 1) & 1) * BST, (t + 1) % T, bx[(t + 1) & 1], w[(t + 1) & 1]);
+      if (s * T + t < nt) compute(bx[t & 1], w[t & 1]);
+      // every LDS read of the slots has returned before they are refilled
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  }
+  __builtin_amdgcn_s_setprio(0);
+  // the rings' last loads (past the wave's share) are not consumed: let them land
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // ---- t[column][row] in LDS: lane (n, h) of band pair p, chunk c holds rows 8 q + 4 h + i of
+  // the pair in acc[4 q + i]
+  const int col = lane & 31;
+  bg_epilogue<CB, NC, WAVES, KL, NR>(g, m, lds, kl, ob, cb, sl, rows, [&](float* reg, int e, bool add) {
+#pragma unroll
+    for (int p = 0; p < RG; ++p)
+#pragma unroll
+      for (int c = 0; c < EC / 32; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float4_t* d = reinterpret_cast<float4_t*>(&reg[(c * 32 + col) * BG_TLS + 32 * p + 8 * q + 4 * h]);
+          const float16_t& a = acc[p][e * (EC / 32) + c];
+          const float4_t v = {a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+          *d = add ? *d + v : v;
+        }
+  });
+}
+
+// ---------------------------------------------------------------- more than 64 columns
+// One workgroup of 4 waves (one per SIMD, up to 512 registers each) per 128-row output block x
+// NB = 16 NC batch columns x k-range, on v_mfma_f32_16x16x32_f16 over tile pairs. The GPU's
+// power limit sets the clock here (1.6 to 1.9 GHz with the matrix cores busy; loops of MFMAs
+// alone hold 1920 TFLOP/s with this shape and 1690 with 32x32x16), so the kernel is built to
+// move and recompute little: a wave holds 64 accumulator tiles, 8 bands x 128 columns with a
+// quarter of the k-range, or 4 bands x 256 columns with half of it, so a fragment of B read
+// from LDS serves 8 or 4 bands, a decoded operand 8 or 16 column chunks, and no fragment of
+// B or word of the stream is read twice by a wave. As above, every wave streams into rings
+// of its own and no barrier is in the loop.
+template <int NC> struct BgWide {
+  static constexpr int WAVES = 4;
+  static constexpr int BW = NC == 8 ? 8 : 4;    // bands per wave
+  static constexpr int KL = BW / 2;             // waves that share a band, each a share of k
+  static constexpr int T = 4;                   // tile columns per stage of packed words (two pairs)
+  static constexpr int PB = NC == 8 ? 3 : 2;    // tile pairs of B in flight (ring slots)
+  static constexpr int NS = 3;                  // stages of packed words in the ring
+};
+
+template <int K, int CB, int V, int NC, int F16, bool SINGLE>
+__global__ __launch_bounds__(256) void bgemm_wide_kernel(LinArgs g) {
+  using Sh = BgWide<NC>;
+  constexpr int BW = Sh::BW, KL = Sh::KL, T = Sh::T, PB = Sh::PB, NS = Sh::NS, WAVES = Sh::WAVES;
+  constexpr int NB = 16 * NC, XQ = NC / 2;      // batch columns, 32-row chunks of B
+  constexpr int NWK = 8 * K, CPT = 2 * K;       // words, 16-byte chunks per tile
+  constexpr int BCH = BW * T * CPT, BL = (BCH + 63) / 64, BST = BL * 256;
+  constexpr int XL = 2 * XQ, XST = XL * 256;    // loads, words of a B slot (one tile pair)
+  constexpr int RING = NS * BST + PB * XST;
+  constexpr bool SUM = F16 || CB == CB_1MAD;    // one fp16 per weight (1MAD: exactly)
+  constexpr int NR = KL, EC = 64;
+  constexpr int WORDS = WAVES * RING > NR * EC * BG_TLS ? WAVES * RING : NR * EC * BG_TLS;
+  static_assert(WORDS <= BG_LDS_WORDS, "rings and epilogue regions fit the LDS");
+  static_assert(PB * XL + 2 * BL < 64, "loads in flight");
+  __shared__ __align__(16) uint32_t lds[WORDS];
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int item = xcd_item(blockIdx.x, g.total);
+  const int mi = SINGLE ? 0 : locate_mat(g, item, false);
+  const LinMat& m = g.m[mi];
+  {
+    // the matrix's fields that the set-up needs, loaded in one round
+    const int f_i0 = m.item0, f_s = m.S, f_t = m.tiles_in, f_n = m.n, f_ob = m.n_ob;
+    const int f_bt = g.batch, f_kr = g.kr;
+    const uint32_t *f_b = m.bits, *f_xf = m.xf;
+    const float *f_sv = m.sv, *f_os = m.osc;
+    asm volatile("" ::"s"(f_i0), "s"(f_s), "s"(f_t), "s"(f_n), "s"(f_ob), "s"(f_bt), "s"(f_kr),
+                 "s"(f_b), "s"(f_xf), "s"(f_sv), "s"(f_os));
+  }
+  // items as in bgemm_kernel
+  const int local = item - m.item0;
+  const int sl = local % m.S, cbob = local / m.S;
+  const int cb = cbob / m.n_ob, ob = cbob % m.n_ob;
+  const int rows = min(128, m.n - ob * 128);
+  const int kl = wave % KL, bg = wave / KL;     // share of the k-range, band group
+  const int ntl = min(g.kr, m.tiles_in - sl * g.kr);
+  const int share = ((ntl + KL - 1) / KL + 1) & ~1;
+  const int j0 = sl * g.kr + kl * share;        // this wave's tile columns j0 .. j0 + nt - 1
+  const int nt = min(share, ntl - kl * share);  // (none: nt <= 0)
+
+  const size_t blk0 = static_cast<size_t>(ob) * 8 * m.tiles_in * NWK;
+  const int nbands = min(8, m.n / 16 - ob * 8);
+  const rsrc_t r_b = make_rsrc(m.bits + blk0, static_cast<unsigned>(nbands * m.tiles_in * NWK * 4));
+  const int nch32 = (g.batch + XF_CHUNK - 1) / XF_CHUNK;
+  const rsrc_t r_x = make_rsrc(reinterpret_cast<const char*>(m.xf) +
+                                   static_cast<size_t>(cb) * XQ * m.tiles_in * XF_FRAG,
+                               static_cast<unsigned>(min(XQ, nch32 - cb * XQ)) * m.tiles_in * XF_FRAG);
+  unsigned boff[BL], bt[BL];
+#pragma unroll
+  for (int q = 0; q < BL; ++q) {
+    const int ch = lane + 64 * q;
+    const int bb = ch / (T * CPT), rem = ch % (T * CPT);
+    bt[q] = rem / CPT;
+    boff[q] = ch < BCH ? static_cast<unsigned>(((BW * bg + bb) * m.tiles_in + j0) * NWK * 4 + rem * 16)
+                       : RSRC_PAST;
+  }
+  uint32_t* ring = lds + wave * RING;
+  const unsigned ring_base = __builtin_amdgcn_readfirstlane(lds_addr(ring));
+  auto load_bits = [&](int s, int slot) {
+#pragma unroll
+    for (int q = 0; q < BL; ++q) {
+      const unsigned o = static_cast<int>(s * T + bt[q]) < nt ? boff[q] + static_cast<unsigned>(s * T * NWK * 4) : RSRC_PAST;
+      load_lds16<false>(r_b, ring_base + static_cast<unsigned>(slot * BST * 4 + q * 1024), o);
+    }
+  };
+  const unsigned xcs = static_cast<unsigned>(m.tiles_in) * XF_FRAG;   // bytes per chunk
+  const unsigned xoff = static_cast<unsigned>(j0) * XF_FRAG + lane * 16;
+  // pair p's fragments: chunk q's two tile columns 1 KB apart; a pair's second column past
+  // the share reads zeros, which its words (any finite weights) then meet
+  auto load_x = [&](int p, int slot) {
+    const unsigned o = 2 * p < nt ? xoff + static_cast<unsigned>(2 * p) * XF_FRAG : RSRC_PAST;
+    const unsigned o1 = 2 * p + 1 < nt ? o : RSRC_PAST;
+#pragma unroll
+    for (int q = 0; q < XQ; ++q)
+      load_lds16_pair(r_x, ring_base + static_cast<unsigned>((NS * BST + slot * XST) * 4 + q * 2048), o + q * xcs, o1 + q * xcs);
+  };
+
+  // lane (r, gq): row r of a band; quads h and h + 2 of the pair's tile gq / 2, h = gq % 2
+  const int r = lane & 15, gq = lane >> 4, h = gq & 1;
+  const QuadPos q0 = quad_pos_v<K, V>(r, h), q1 = quad_pos_v<K, V>(r, h + 2);
+  const uint32_t* wbase = ring + (gq >> 1) * NWK;
+  const uint32_t* xbase = ring + NS * BST + (gq >> 1) * 256 + h * 128 + r * 4;
+  float4_t acc[BW][NC];
+#pragma unroll
+  for (int b = 0; b < BW; ++b)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[b][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+  asm volatile("" ::: "memory");
+
+  load_bits(0, 0);
+  load_bits(1, 1);
+#pragma unroll
+  for (int p = 0; p < PB; ++p) load_x(p, p);
+  u32x4_t bx[2][NC];
+  uint32_t w[2][BW][4];
+  auto read_pair = [&](int bslot, int t2, int xslot, u32x4_t (&b)[NC], uint32_t (&v)[BW][4]) {
+    const uint32_t* xp = xbase + xslot * XST;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      b[c] = *reinterpret_cast<const u32x4_t*>(xp + (c >> 1) * 512 + (c & 1) * 64);
+    const uint32_t* wp = wbase + bslot * BST;
+#pragma unroll
+    for (int i = 0; i < BW; ++i) {
+      const uint32_t* tp = wp + (i * T + 2 * t2) * NWK;
+      v[i][0] = tp[q0.wa];
+      v[i][1] = tp[q0.wb];
+      v[i][2] = tp[q1.wa];
+      v[i][3] = tp[q1.wb];
+    }
+  };
+  auto compute = [&](const u32x4_t (&b)[NC], const uint32_t (&v)[BW][4]) {
+    // band i + 1 is decoded between the MFMAs of band i
+    half8_t hi[2], lo[2];
+    auto operands = [&](int i) {
+      uint32_t p0[4], p1[4];
+      decode_lcg<K, CB, V>(v[i][0], v[i][1], q0.sh, p0);
+      decode_lcg<K, CB, V>(v[i][2], v[i][3], q1.sh, p1);
+      if constexpr (SUM)
+        hi[i & 1] = operand_sum<CB>(p0, p1);
+      else
+        operand_planes(p0, p1, hi[i & 1], lo[i & 1]);
+    };
+    operands(0);
+#pragma unroll
+    for (int i = 0; i < BW; ++i) {
+      if (i + 1 < BW) operands(i + 1);
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[i & 1], __builtin_bit_cast(half8_t, b[c]), acc[i][c], 0, 0, 0);
+      if constexpr (!SUM) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[i & 1], __builtin_bit_cast(half8_t, b[c]), acc[i][c], 0, 0, 0);
+      }
+      if (i + 1 < BW) {
+        constexpr int M = SUM ? NC : 2 * NC, VPM = (40 + M - 1) / M;
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);     // an MFMA
+          __builtin_amdgcn_sched_group_barrier(0x2, VPM, 0);   // VALU operations
+        }
+      }
+    }
+  };
+  // loads land in issue order: pair 0's fragments (and stages 0 and 1 before them)
+  wait_vmcnt<(PB - 1) * XL>();
+  asm volatile("" ::: "memory");
+  read_pair(0, 0, 0, bx[0], w[0]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const int nst = (nt + T - 1) / T;
+  int bs = 0, xs = 0;                           // ring slots of stage s and pair p
+  for (int s = 0; s < nst; ++s) {
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      // the slots refilled here were read into registers before, and those reads returned:
+      // stage s - 1's words and pair p's fragments
+      if (t2 == 0) load_bits(s + 2, bs >= 1 ? bs - 1 : NS - 1);
+      load_x(2 * s + t2 + PB, xs);
+      // after pair p + 1's fragments (and its stage's words before them) came PB - 1 pairs of
+      // fragments and a stage of words, if one was issued in the last PB - 1 pairs
+      if (PB == 3 || t2 == 0)
+        wait_vmcnt<(PB - 1) * XL + BL>();
+      else
+        wait_vmcnt<(PB - 1) * XL>();
+      asm volatile("" ::: "memory");
+      xs = xs + 1 < PB ? xs + 1 : 0;
+      if (t2 == 1) bs = bs + 1 < NS ? bs + 1 : 0;
+      read_pair(bs, (t2 + 1) & 1, xs, bx[(t2 + 1) & 1], w[(t2 + 1) & 1]);
+      if (s * T + 2 * t2 < nt) compute(bx[t2], w[t2]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  bg_epilogue<CB, NC, WAVES, KL, NR>(g, m, lds, kl, ob, cb, sl, rows, [&](float* reg, int e, bool add) {
+#pragma unroll
+    for (int i = 0; i < BW; ++i)
+#pragma unroll
+      for (int c = 0; c < EC / 16; ++c) {
+        float4_t* d = reinterpret_cast<float4_t*>(&reg[(c * 16 + r) * BG_TLS + 16 * (BW * bg + i) + 4 * gq]);
+        const float4_t v = acc[i][e * (EC / 16) + c];
+        *d = add ? *d + v : v;
+      }
+  });
 }
 
 // Split-K reduction of bgemm_kernel: one wave per (matrix, 128-row block, batch column):

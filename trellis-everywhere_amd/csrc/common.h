@@ -23,6 +23,7 @@ constexpr int MAX_GROUP = 8;   // linears per launch
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 // Launch arguments. The kernels read them straight from the kernel-argument segment, which is
@@ -56,6 +57,7 @@ struct alignas(64) LinMat {
   uint32_t* xf;         // workspace: [batch][xfw words] folded activations (xfold_kernel)
   int chunk0;           // first group-wide x-fold job of this matrix
   int fold0;            // first group-wide bfold_kernel job of this matrix
+  int y_words;          // every row of y starts at a 4-byte aligned address
 };
 
 struct alignas(64) LinArgs {
@@ -77,6 +79,7 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, unsigned bytes) {
                                            0x00020000);
 }
 constexpr unsigned RSRC_OOB = 0x40000000u;   // an offset past every buffer made here
+constexpr unsigned RSRC_PAST = 0x80000000u;  // the same for buffers of up to 2 GiB
 constexpr int AUX_NT = 2;                    // nontemporal cache policy (gfx94x/gfx950)
 constexpr int AUX_SC1 = 16;                  // agent scope (sc1): written through past the L2
 
@@ -97,10 +100,24 @@ __device__ __forceinline__ void st_wt(_Float16* p, _Float16 v) {
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// 16 bytes at a 4-byte aligned address, written through like st_wt. (The s_nop: gfx9 needs a
+// wait state between a store of more than 8 bytes and a VALU write of its data registers, and
+// the compiler's hazard pass does not look inside inline assembly.)
+__device__ __forceinline__ void st_wt16(void* p, u32x4_t v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+}
+
 // LDS byte address of a shared-memory pointer.
 __device__ __forceinline__ unsigned lds_addr(const void* p) {
   return static_cast<unsigned>(reinterpret_cast<size_t>(
       (__attribute__((address_space(3))) void*)(const_cast<void*>(p))));
+}
+
+// A workgroup barrier for what waves exchange through LDS: their LDS accesses are complete, but
+// stores to memory may still be in flight (__syncthreads waits for their acknowledgements too,
+// 1 us and more for write-through stores).
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // s_waitcnt for the vector-memory counter only (expcnt and lgkmcnt at their maxima)
@@ -120,16 +137,45 @@ __device__ __forceinline__ void wait_vmcnt() {
 // correct (they may wait longer than needed, never shorter). GFX9 needs one wait state
 // between an SALU write of M0 and an LDS-DMA load that reads it; the compiler's hazard
 // pass does not look inside inline assembly, so the s_nop is written here.
+// NT: nontemporal, for words that are read once (kept out of the way in the L2).
+template <bool NT = true>
 __device__ __forceinline__ void load_lds16(rsrc_t r, unsigned lds_base, unsigned voff) {
+  unsigned saved;
+  if constexpr (NT)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %3, 0 offen nt lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "s"(lds_base), "v"(voff), "s"(r)
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "s"(lds_base), "v"(voff), "s"(r)
+        : "memory");
+}
+
+// Two such loads 1 KB apart in LDS and in the buffer, at byte offsets v0 and v1 + 1024 (v1 = v0,
+// or out of range on its own).
+__device__ __forceinline__ void load_lds16_pair(rsrc_t r, unsigned lds_base, unsigned v0, unsigned v1) {
   unsigned saved;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %1\n\t"
       "s_nop 0\n\t"
-      "buffer_load_dwordx4 %2, %3, 0 offen nt lds\n\t"
+      "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
+      "buffer_load_dwordx4 %3, %4, 0 offen offset:1024 lds\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(saved)
-      : "s"(lds_base), "v"(voff), "s"(r)
+      : "s"(lds_base), "v"(v0), "v"(v1), "s"(r)
       : "memory");
 }
 
@@ -340,19 +386,94 @@ __device__ __forceinline__ int xf_pair_slot(int e) {
 }
 
 // ---------------------------------------------------------------- x fold
-// xf = Hb_k(isc * su * x) scaled by 1/sqrt(block_in), stored as (x,x) fp16 pairs. One
-// wave per (matrix, group of R batch rows, 128-column chunk), every load a range-checked
-// buffer load issued up front. Up to 64 rows the kernel is latency-bound (a few MB): one
-// row per wave gives every SIMD several waves to overlap the transform's dependent lane
-// exchanges (8B gate+up fold at batch 64, alone in a graph chain: 2.7 us per launch,
-// against 2.9 with 2 rows and 3.6 with 4 rows per wave). From 256 rows up a launch needs
-// several rounds of waves on the CUs, each paying the start-up latency: four rows per wave
-// (their scales loaded once, the rows transformed together) took the 8B block's folds at
-// batch 512 from 12.5 to 9.5 us per launch on average (kernel trace), eight rows 9.7; the
-// block 517 -> 503.5 us, 360 -> 347.5 in the fp16-weight mode; at 128 rows no change.
-__host__ __device__ constexpr int xfold_rows(int batch) { return batch >= 256 ? 4 : 1; }
+// xf = Hb_k(isc * su * x) scaled by 1/sqrt(block_in), once per batched call.
+//
+// Above 16 rows, the kernels' B layout: chunks of 32 batch rows, each
+// [tile column][h = 0, 1][32 rows] of 16 bytes holding the fp16 values of columns 4h .. 4h+3
+// and 8+4h .. 8+4h+3 of the tile: the 1 KB of a (chunk, tile column) is one fragment of
+// v_mfma_f32_32x32x16_f16, lane l = (row l % 32, h = l / 32), read as one coalesced load.
+constexpr int XF_CHUNK = 32;          // batch rows per chunk
+constexpr int XF_FRAG = 1024;         // bytes per (chunk, tile column)
+// batch rows per x-fold job: one for the 16-row kernel's layout; above, a workgroup's 8, or 32
+// (four per wave, their scales loaded once and the rows transformed together) from 256 rows
+// up, where a launch needs several rounds of waves on the CUs, each paying the start-up latency
+// (8B block at 512 rows 517 -> 503.5 us; at 128 rows no change)
+__host__ __device__ constexpr int xfold_rows(int nc, int batch) { return nc == 1 ? 1 : batch >= 256 ? 32 : 8; }
 #ifdef TRELLIS_XFOLD_DEFINE
-template <int XFOLD_ROWS, bool SINGLE>
+// The x fold into that layout. One wave per R batch rows (8 apart) of a group of 8 R, all of
+// one 128-column chunk, so a workgroup of 8 waves holds runs of 8 R rows of each 16-byte
+// unit: the values meet in LDS and go out as 128-byte (R = 1) to 512-byte (R = 4) runs. Rows
+// of the last chunk past the call's are not written (they feed only MFMA columns that are
+// never stored).
+template <int R, bool SINGLE>
+__global__ __launch_bounds__(512) void xfold_frag_kernel(LinArgs g) {
+  constexpr int ROWS = 8 * R;
+  constexpr int TH = ROWS * 16 + 16;   // bytes per (tile column, h) in LDS (+16: bank spread)
+  __shared__ __align__(16) unsigned char buf[16 * TH];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int mi = SINGLE ? 0 : locate_mat(g, blockIdx.x, true);
+  const LinMat& m = g.m[mi];
+  const int local = blockIdx.x - m.chunk0;
+  const int nch = (m.k + 127) / 128;
+  const int rg = local / nch, ch = local % nch;
+  const int b0 = rg * ROWS;
+  const int kvalid = min(128, m.k - ch * 128);
+  const int xsh = g.x_f16 ? 1 : 2;
+  const rsrc_t r_x = make_rsrc(m.x, static_cast<unsigned>((g.batch - 1) * m.ldx + m.k) << xsh);
+  const rsrc_t r_su = make_rsrc(m.su, m.k * 4), r_isc = make_rsrc(m.isc, m.k * 4);
+  const int e0 = ch * 128 + lane, e1 = e0 + 64;
+  const float s0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_su, e0 * 4, 0, 0)) *
+                   __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_isc, e0 * 4, 0, 0));
+  const float s1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_su, e1 * 4, 0, 0)) *
+                   __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_isc, e1 * 4, 0, 0));
+  uint32_t w0[R], w1[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    // a row past the call's repeats its last one, a column past the matrix reads zeros
+    const unsigned row = static_cast<unsigned>(min(b0 + wave + 8 * r, g.batch - 1) * m.ldx);
+    const unsigned o0 = ((row + e0) << xsh) & ~3u, o1 = ((row + e1) << xsh) & ~3u;
+    w0[r] = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(e0 < m.k ? o0 : RSRC_PAST), 0, 0);
+    w1[r] = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(e1 < m.k ? o1 : RSRC_PAST), 0, 0);
+  }
+  const float nrm = m.nrm_in;
+  const FwhtLane fl = fwht_lane(lane, m.block_in);
+  float lov[R], hiv[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    lov[r] = lane < kvalid ? act_value(w0[r], e0, g.x_f16) * s0 : 0.0f;
+    hiv[r] = lane + 64 < kvalid ? act_value(w1[r], e1, g.x_f16) * s1 : 0.0f;
+  }
+  fwht_chunks<R>(lov, hiv, m.block_in, lane, fl);
+  // column e: tile e / 16, quad q4 = (e / 4) % 4 -> h = q4 % 2, half 4 (q4 / 2) + e % 4
+  unsigned char* dst = buf + (2 * (lane >> 4) + ((lane >> 2) & 1)) * TH + 8 * ((lane >> 3) & 1) + 2 * (lane & 3);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int n = wave + 8 * r;
+    *reinterpret_cast<_Float16*>(dst + n * 16) = static_cast<_Float16>(lov[r] * nrm);
+    *reinterpret_cast<_Float16*>(dst + 8 * TH + n * 16) = static_cast<_Float16>(hiv[r] * nrm);
+  }
+  __syncthreads();
+  const rsrc_t r_o = make_rsrc(reinterpret_cast<char*>(m.xf) + static_cast<size_t>(b0 / XF_CHUNK) * m.tiles_in * XF_FRAG,
+                               static_cast<unsigned>(m.tiles_in) * XF_FRAG);
+#pragma unroll
+  for (int i = 0; i < (16 * ROWS + 511) / 512; ++i) {
+    const int u = threadIdx.x + 512 * i;
+    const int th = u / ROWS, n = u % ROWS;
+    // tile columns past the matrix fall outside the chunk
+    if (u < 16 * ROWS && b0 + n < g.batch) {
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(buf + th * TH + n * 16);
+      const unsigned o = (static_cast<unsigned>(ch * 16 + th) * XF_CHUNK + b0 % XF_CHUNK + n) * 16;
+      __builtin_amdgcn_raw_buffer_store_b128(v, r_o, static_cast<int>(o), 0, AUX_SC1);
+    }
+  }
+}
+
+// The x fold for the 16-row kernel: rows of (x, x) fp16 pairs, or in the fp16-weight mode of
+// fp16 values in tile-pair order (xf_pair_slot). One wave per (matrix, batch row, 128-column
+// chunk), every load a range-checked buffer load issued up front: a few rows are latency-
+// bound, and one row per wave gives every SIMD several waves to overlap the transform's
+// dependent lane exchanges.
+template <bool SINGLE>
 __global__ __launch_bounds__(256) void xfold_kernel(LinArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int job = blockIdx.x * 4 + wave;
@@ -362,8 +483,7 @@ __global__ __launch_bounds__(256) void xfold_kernel(LinArgs g) {
   const LinMat& m = g.m[mi];
   const int local = job - m.chunk0;
   const int nch = (m.k + 127) / 128;
-  const int rg = local / nch, ch = local % nch;
-  const int b0 = rg * XFOLD_ROWS;
+  const int b0 = local / nch, ch = local % nch;
   const int kvalid = min(128, m.k - ch * 128);
   const int xsh = g.x_f16 ? 1 : 2;
   const rsrc_t r_x = make_rsrc(m.x, static_cast<unsigned>(g.batch) * static_cast<unsigned>(m.ldx) << xsh);
@@ -373,41 +493,24 @@ __global__ __launch_bounds__(256) void xfold_kernel(LinArgs g) {
                    __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_isc, e0 * 4, 0, 0));
   const float s1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_su, e1 * 4, 0, 0)) *
                    __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_isc, e1 * 4, 0, 0));
-  uint32_t w0[XFOLD_ROWS], w1[XFOLD_ROWS];
-#pragma unroll
-  for (int r = 0; r < XFOLD_ROWS; ++r) {
-    const unsigned row = static_cast<unsigned>((b0 + r) * m.ldx);
-    w0[r] = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e0) << xsh) & ~3u), 0, 0);
-    w1[r] = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e1) << xsh) & ~3u), 0, 0);
-  }
+  const unsigned row = static_cast<unsigned>(b0 * m.ldx);
+  const uint32_t w0 = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e0) << xsh) & ~3u), 0, 0);
+  const uint32_t w1 = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e1) << xsh) & ~3u), 0, 0);
   const float nrm = m.nrm_in;
-  const FwhtLane fl = fwht_lane(lane, m.block_in);
-  // the rows are transformed together, level by level, so their dependent lane exchanges
-  // overlap (rows past the call's were loaded as zeros and are not stored)
-  float lov[XFOLD_ROWS], hiv[XFOLD_ROWS];
-#pragma unroll
-  for (int r = 0; r < XFOLD_ROWS; ++r) {
-    // an f16 row stride is even, so the element's half within its word follows e
-    lov[r] = lane < kvalid ? act_value(w0[r], e0, g.x_f16) * s0 : 0.0f;
-    hiv[r] = lane + 64 < kvalid ? act_value(w1[r], e1, g.x_f16) * s1 : 0.0f;
-  }
-  fwht_chunks<XFOLD_ROWS>(lov, hiv, m.block_in, lane, fl);
-#pragma unroll
-  for (int r = 0; r < XFOLD_ROWS; ++r) {
-    if (b0 + r >= g.batch) break;
-    const float lo = lov[r], hi = hiv[r];
-    if (g.mma_f16) {
-      // fp16 values in tile-pair order (xf_pair_slot); columns k .. kp - 1 of the last
-      // pair are written as zeros (lo and hi are zero there)
-      _Float16* dst = reinterpret_cast<_Float16*>(m.xf + static_cast<size_t>(b0 + r) * m.xfw);
-      const int kp = 2 * m.xfw;
-      if (e0 < kp) st_wt(dst + xf_pair_slot(e0), static_cast<_Float16>(lo * nrm));
-      if (e1 < kp) st_wt(dst + xf_pair_slot(e1), static_cast<_Float16>(hi * nrm));
-    } else {
-      uint32_t* dst = m.xf + static_cast<size_t>(b0 + r) * m.xfw + ch * 128;
-      if (lane < kvalid) st_wt(dst + lane, dup_half(lo * nrm));
-      if (lane + 64 < kvalid) st_wt(dst + lane + 64, dup_half(hi * nrm));
-    }
+  // an f16 row stride is even, so the element's half within its word follows e
+  float lo = lane < kvalid ? act_value(w0, e0, g.x_f16) * s0 : 0.0f;
+  float hi = lane + 64 < kvalid ? act_value(w1, e1, g.x_f16) * s1 : 0.0f;
+  fwht_chunk(lo, hi, m.block_in, lane);
+  if (g.mma_f16) {
+    // columns k .. kp - 1 of the last pair are written as zeros (lo and hi are zero there)
+    _Float16* dst = reinterpret_cast<_Float16*>(m.xf + static_cast<size_t>(b0) * m.xfw);
+    const int kp = 2 * m.xfw;
+    if (e0 < kp) st_wt(dst + xf_pair_slot(e0), static_cast<_Float16>(lo * nrm));
+    if (e1 < kp) st_wt(dst + xf_pair_slot(e1), static_cast<_Float16>(hi * nrm));
+  } else {
+    uint32_t* dst = m.xf + static_cast<size_t>(b0) * m.xfw + ch * 128;
+    if (lane < kvalid) st_wt(dst + lane, dup_half(lo * nrm));
+    if (lane + 64 < kvalid) st_wt(dst + lane + 64, dup_half(hi * nrm));
   }
 }
 #endif
@@ -466,6 +569,66 @@ __device__ __forceinline__ half8_t decode_a_pair(uint32_t wlo0, uint32_t whi0, u
     o[1] = add_halves2(a0[2], a0[3]);
     o[2] = add_halves2(a1[0], a1[1]);
     o[3] = add_halves2(a1[2], a1[3]);
+  }
+  return __builtin_bit_cast(half8_t, o);
+}
+
+// The A operands of v_mfma_f32_32x32x16_f16 for one tile column of a band pair: lane l = (row
+// l % 32 of the pair, h = l / 32) holds the 8 weights of the tile's quads h and h + 2, in B's
+// order (XF_FRAG). LCG values p0 (quad h) and p1 (quad h + 2).
+//
+// operand_sum: each codebook value as one fp16. MCG / 3INST: the rounded sum of the halves
+// (the fp16-weight mode). 1MAD: byte sum - 510, exact: sad accumulates onto 0x6400 (1024 as
+// fp16, one unit per integer up to 2047) in each half, minus 1534.
+template <int CB>
+__device__ __forceinline__ half8_t operand_sum(const uint32_t (&p0)[4], const uint32_t (&p1)[4]) {
+  uint32_t o[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const uint32_t a = w < 2 ? p0[2 * w] : p1[2 * w - 4], b = w < 2 ? p0[2 * w + 1] : p1[2 * w - 3];
+    if constexpr (CB == CB_1MAD) {
+      const uint32_t y = __builtin_amdgcn_sad_hi_u8(b, 0u, __builtin_amdgcn_sad_u8(a, 0u, 0x64006400u));
+      const half2_t off = {static_cast<_Float16>(-1534.0f), static_cast<_Float16>(-1534.0f)};
+      o[w] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, y) + off);
+    } else {
+      o[w] = add_halves2(lop3_pair(a), lop3_pair(b));
+    }
+  }
+  return __builtin_bit_cast(half8_t, o);
+}
+
+// MCG / 3INST, exact: the high and the low halves of the 8 weights as two operands against
+// the same B fragment; their products' sum is (hi + lo) * x.
+__device__ __forceinline__ void operand_planes(const uint32_t (&p0)[4], const uint32_t (&p1)[4],
+                                               half8_t& hi, half8_t& lo) {
+  uint32_t h[4], l[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const uint32_t a = w < 2 ? p0[2 * w] : p1[2 * w - 4], b = w < 2 ? p0[2 * w + 1] : p1[2 * w - 3];
+    h[w] = lop3_pair(__builtin_amdgcn_perm(b, a, 0x07060302u));
+    l[w] = lop3_pair(__builtin_amdgcn_perm(b, a, 0x05040100u));
+  }
+  hi = __builtin_bit_cast(half8_t, h);
+  lo = __builtin_bit_cast(half8_t, l);
+}
+
+// MCG / 3INST, exact: one quad's (hi, lo) pairs as they come, against a duplicated fragment
+// (dup_frag).
+__device__ __forceinline__ half8_t operand_pairs(const uint32_t (&p)[4]) {
+  uint32_t o[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) o[q] = lop3_pair(p[q]);
+  return __builtin_bit_cast(half8_t, o);
+}
+
+// A B fragment's quad h (half 0) or h + 2 (half 1) with every value twice.
+__device__ __forceinline__ half8_t dup_frag(u32x4_t b, int half) {
+  uint32_t o[4];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const uint32_t v = b[2 * half + q];
+    o[2 * q] = __builtin_amdgcn_perm(v, v, 0x01000100u);
+    o[2 * q + 1] = __builtin_amdgcn_perm(v, v, 0x03020302u);
   }
   return __builtin_bit_cast(half8_t, o);
 }

@@ -117,21 +117,29 @@ __device__ __forceinline__ uint32_t cb_out(uint32_t p) {
     return lop3_pair(p);
 }
 
-// Raw codebook outputs (cb_raw) of the lane's four weights (columns 4g..4g+3).
+// LCG values (before the output stage, cb_out) of the lane's four weights (columns 4g..4g+3).
 template <int K, int CB, int V = 1>
-__device__ __forceinline__ void decode_quad(uint32_t wlo, uint32_t whi, int sh, uint32_t (&raw)[4]) {
+__device__ __forceinline__ void decode_lcg(uint32_t wlo, uint32_t whi, int sh, uint32_t (&p)[4]) {
   const uint32_t u = __builtin_amdgcn_alignbit(whi, wlo, sh);
   if constexpr (V == 2) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint32_t p = lcg_p<CB>((u >> (2 * K * (1 - h))) & 0xFFFFu);
-      raw[2 * h] = cb_out<CB>(p);
-      raw[2 * h + 1] = cb_out<CB>(p * Lcg<CB>::MUL + Lcg<CB>::ADD);
+      p[2 * h] = lcg_p<CB>((u >> (2 * K * (1 - h))) & 0xFFFFu);
+      p[2 * h + 1] = p[2 * h] * Lcg<CB>::MUL + Lcg<CB>::ADD;
     }
   } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) raw[q] = cb_raw<CB>((u >> (K * (3 - q))) & 0xFFFFu);
+    for (int q = 0; q < 4; ++q) p[q] = lcg_p<CB>((u >> (K * (3 - q))) & 0xFFFFu);
   }
+}
+
+// Raw codebook outputs (cb_raw) of the lane's four weights (columns 4g..4g+3).
+template <int K, int CB, int V = 1>
+__device__ __forceinline__ void decode_quad(uint32_t wlo, uint32_t whi, int sh, uint32_t (&raw)[4]) {
+  uint32_t p[4];
+  decode_lcg<K, CB, V>(wlo, whi, sh, p);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) raw[q] = cb_out<CB>(p[q]);
 }
 
 }  // namespace trellis

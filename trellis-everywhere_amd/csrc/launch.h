@@ -19,8 +19,8 @@ constexpr int gemv_nb(int batch) { return batch <= 1 ? 1 : batch == 2 ? 2 : batc
 template <int K>
 int launch_gemv_k(int cb, int V, int kc, const LinArgs& g, hipStream_t st);
 
-// bgemm_kernel<K, cb, V, nc, g.mma_f16> over g.total items (the x fold has been launched
-// before it).
+// The batched kernel for column blocks of 16 nc (bgemm16_kernel, bgemm_kernel,
+// bgemm_wide_kernel) over g.total items (the x fold has been launched before it).
 template <int K>
 int launch_bgemm_k(int cb, int V, int nc, const LinArgs& g, hipStream_t st);
 
@@ -46,9 +46,13 @@ static int launch_bfold_cb(int nc, int nfold, const LinArgs& g, hipStream_t st) 
       if (one) hipLaunchKernelGGL((bfold_kernel<CB, 4, true>), grid, dim3(256), 0, st, g);
       else hipLaunchKernelGGL((bfold_kernel<CB, 4, false>), grid, dim3(256), 0, st, g);
       break;
-    default:
+    case 8:
       if (one) hipLaunchKernelGGL((bfold_kernel<CB, 8, true>), grid, dim3(256), 0, st, g);
       else hipLaunchKernelGGL((bfold_kernel<CB, 8, false>), grid, dim3(256), 0, st, g);
+      break;
+    default:
+      if (one) hipLaunchKernelGGL((bfold_kernel<CB, 16, true>), grid, dim3(256), 0, st, g);
+      else hipLaunchKernelGGL((bfold_kernel<CB, 16, false>), grid, dim3(256), 0, st, g);
       break;
   }
   return hipGetLastError() == hipSuccess ? 0 : 13;
@@ -109,14 +113,17 @@ template <int K, int CB, int V, int F16>
 static int launch_bgemm_nc(int nc, const LinArgs& g, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(g.total));
   const bool one = g.nmat == 1;
-#define TRELLIS_BG_LAUNCH(NCV) \
-  if (one) hipLaunchKernelGGL((bgemm_kernel<K, CB, V, NCV, F16, true>), grid, dim3(64 * BgWaves<NCV, F16>::WV), 0, st, g); \
-  else hipLaunchKernelGGL((bgemm_kernel<K, CB, V, NCV, F16, false>), grid, dim3(64 * BgWaves<NCV, F16>::WV), 0, st, g);
+  // 1MAD's values are exact in one fp16: above 16 columns its exact mode is the fp16-weight one
+  constexpr int F = CB == CB_1MAD ? 1 : F16;
+#define TRELLIS_BG_LAUNCH(KERNEL, THREADS, ...) \
+  if (one) hipLaunchKernelGGL((KERNEL<K, CB, V, __VA_ARGS__, true>), grid, dim3(THREADS), 0, st, g); \
+  else hipLaunchKernelGGL((KERNEL<K, CB, V, __VA_ARGS__, false>), grid, dim3(THREADS), 0, st, g);
   switch (nc) {
-    case 1: TRELLIS_BG_LAUNCH(1) break;
-    case 2: TRELLIS_BG_LAUNCH(2) break;
-    case 4: TRELLIS_BG_LAUNCH(4) break;
-    default: TRELLIS_BG_LAUNCH(8) break;
+    case 1: TRELLIS_BG_LAUNCH(bgemm16_kernel, 1024, F16) break;
+    case 2: TRELLIS_BG_LAUNCH(bgemm_kernel, 512, 2, F) break;
+    case 4: TRELLIS_BG_LAUNCH(bgemm_kernel, 512, 4, F) break;
+    case 8: TRELLIS_BG_LAUNCH(bgemm_wide_kernel, 256, 8, F) break;
+    default: TRELLIS_BG_LAUNCH(bgemm_wide_kernel, 256, 16, F) break;
   }
 #undef TRELLIS_BG_LAUNCH
   return hipGetLastError() == hipSuccess ? 0 : 13;

@@ -1,7 +1,7 @@
 // trellis_amd.hip — C ABI (include/trellis_amd.h): validation, launch planning, the
 // bit-exact tile decode kernel and the dispatch to the decode-matmul kernels (gemv_kernel at
-// batch 1 to 4 and, where use_gemv picks it, 5 to 16; xfold_kernel + bgemm_kernel
-// (+ bfold_kernel) otherwise).
+// batch 1 to 4 and, where use_gemv picks it, 5 to 16; an x fold + a batched kernel (+ bfold_kernel)
+// otherwise).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -163,34 +163,47 @@ int gemv_kr(const trellis_desc* const* W, int count, int batch) {
   return best;
 }
 
-// Batch >= 2 (bgemm_kernel): NC 16-column batch chunks per workgroup (up to 128 columns),
-// a work item is one 128-row block x one column block x one k-range of kr tile columns
-// (a multiple of the k-step: 16 tiles at 16 columns, 8 up to 64 and in the fp16-weight
-// mode, else 6), run by one workgroup per CU (16 waves; 12 for the exact mode's 128-column
-// blocks). kr minimises ceil(items/CUs) x the per-SIMD work of an item (2 bands x kr tiles
-// x (decode ~61 + NC MFMAs x ~19 cycles; fp16-weight mode ~75 + NC x ~10; ~225 for the
-// exact mode's 128-column blocks at three waves per SIMD, fitted to a sweep of both widths
-// on the 8B block's launches at 128-512 rows, where it picks the faster width for all but
-// q/k/v at 128 and 192 rows, ~3 us each)) plus, with split-K,
-// the bfold_kernel launch (~1.5 us) and the partial blocks it moves (S x rows x NB x 4
-// bytes written and read at ~2.5 KB per cycle), plus a start-up latency per round after
-// the first. TRELLIS_BGEMM_KR forces a value, TRELLIS_BGEMM_NC the column-block width.
-static int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bool f16,
-                         long long* cost) {
+// The batched kernels (bgemm.h): NC 16-column batch chunks per workgroup, a work item being one
+// 128-row block x one column block x one k-range of kr tile columns, a multiple of the
+// kernel's step (16 tiles for the 16-row kernel in the exact mode, else 8: a tile per wave at
+// 32 and 64 columns, a pair at 128). The model of a launch, in ns: rounds of items over the
+// CUs x (2 kr band-tiles per SIMD x the time of one + what an item costs besides: start-up,
+// the k-lanes' meeting, output fold), plus, with split-K, the bfold_kernel launch and the
+// partial blocks it moves. The constants follow the kernels' stamped loops and a sweep of
+// every width on the 8B block's launches and a 2048 x 2048 layer at 48 to 2048 rows in both
+// modes, where the width chosen is on average 0.8 % slower than the fastest one (at worst
+// 13 %: q/k/v at 512 rows in the fp16-weight mode). TRELLIS_BGEMM_KR forces a k-range,
+// TRELLIS_BGEMM_NC the width.
+struct BgCost {
+  int tile, item;   // ns per band-tile and SIMD, ns per item
+};
+BgCost bgemm_cost(int nc, bool sum) {
+  // sum: one fp16 per weight (the fp16-weight mode, 1MAD); above 64 columns two MACs per
+  // weight cost their time, up to 64 the decode and its issue set it
+  switch (nc) {
+    case 1: return {33, 2600};
+    case 2: return sum ? BgCost{38, 3000} : BgCost{40, 3000};
+    case 4: return sum ? BgCost{50, 6000} : BgCost{58, 6100};
+    case 8: return sum ? BgCost{76, 8700} : BgCost{93, 8800};
+    default: return sum ? BgCost{116, 18000} : BgCost{150, 18000};
+  }
+}
+
+// Largest k-range with `split` off: one per block.
+int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool split,
+                  long long* cost) {
   int maxt = 0;
   for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
-  const int kt = f16 ? 8 : nc == 1 ? 16 : nc <= 4 ? 8 : 6;   // BgStep<nc, f16>::KT
-  // per band-tile SIMD cycles: the decode and NC MFMAs (the fp16-weight mode decodes a
-  // little more and issues half the MFMAs)
-  const long long tile_cost = f16 ? 75 + 10 * nc : nc == 8 ? 225 : 61 + 19 * nc;
+  const int kt = nc == 1 && !f16 ? 16 : 8;
+  const BgCost bc = bgemm_cost(nc, f16 || W[0]->codebook == TRELLIS_CB_1MAD);
   const int cap = ((maxt + kt - 1) / kt) * kt;
   const long long cus = device_cus();
   const long long ncb = (batch + 16 * nc - 1) / (16 * nc);
   const int forced = env_int("TRELLIS_BGEMM_KR", 0);
-  const bool force = forced >= kt && forced % kt == 0;
+  const bool force = split && forced >= kt && forced % kt == 0;
   int best = cap;
   long long best_cost = -1;
-  for (int kr = force ? (forced < cap ? forced : cap) : kt; kr <= cap; kr += kt) {
+  for (int kr = !split ? cap : force ? (forced < cap ? forced : cap) : kt; kr <= cap; kr += kt) {
     long long items = 0, part_bytes = 0;
     int smax = 1;
     for (int i = 0; i < count; ++i) {
@@ -202,8 +215,8 @@ static int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int
     }
     if (smax > 16 && !force) continue;
     const long long rounds = (items + cus - 1) / cus;
-    const long long epi = smax > 1 ? 3600 + 2 * part_bytes / 2500 : 0;
-    const long long c = rounds * kr * 2 * tile_cost + epi + (rounds - 1) * 3600;
+    const long long c = rounds * (2LL * kr * bc.tile + bc.item) +
+                        (smax > 1 ? 3500 + part_bytes / 4500 : 0);
     if (best_cost < 0 || c < best_cost) {
       best = kr;
       best_cost = c;
@@ -214,28 +227,32 @@ static int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int
   return best;
 }
 
-int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f16) {
+int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool split) {
   long long cost;
-  return bgemm_kr_cost(W, count, batch, nc, f16, &cost);
+  return bgemm_kr_cost(W, count, batch, nc, f16, split, &cost);
 }
 
-// Column-block width: 16, 32 or 64 columns up to batch 64; above, the fp16-weight mode
-// takes 128, and the exact mode 64 (four waves per SIMD) or 128 (three waves per SIMD, each
-// tile decoded half as often), whichever the cost model above finds cheaper for the group
-// (8B block at batch 512: q/k/v and gate+up at 128 columns, 100 -> 87 and 277 -> 243 us;
-// o stays at 64, where 128 measured 53 -> 57 us; one gate projection at batch 96 stays at 64,
-// at 256 takes 128: 92 -> 76 us).
+// Column-block width in 16-column units: 1 up to 16 rows, 2 up to 32; above, the width that
+// the model above finds cheapest for the group, of 32 and 64 columns up to 64 rows (at 64
+// rows the 8B o launch takes 17.5 us in 32-column blocks and 19.7 in 64-column ones, gate+up
+// 53.7 and 40.8), else of 64, 128 and 256 (gate+up at 512 rows 246, 205 and 222 us, at 1024
+// rows 472, 395 and 365; o at 256 rows 33.0, 33.5 and 39.5).
 int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16) {
   const int forced = env_int("TRELLIS_BGEMM_NC", 0);
-  if (forced == 1 || forced == 2 || forced == 4 || forced == 8) return forced;
+  if (forced == 1 || forced == 2 || forced == 4 || forced == 8 || forced == 16) return forced;
   if (batch <= 16) return 1;
   if (batch <= 32) return 2;
-  if (batch <= 64) return 4;
-  if (f16) return 8;
-  long long c4, c8;
-  bgemm_kr_cost(W, count, batch, 4, false, &c4);
-  bgemm_kr_cost(W, count, batch, 8, false, &c8);
-  return c8 < c4 ? 8 : 4;
+  int best = 0;
+  long long best_cost = 0;
+  for (int nc = batch <= 64 ? 2 : 4; nc <= (batch <= 64 ? 4 : 16); nc *= 2) {
+    long long c;
+    bgemm_kr_cost(W, count, batch, nc, f16, true, &c);
+    if (best == 0 || c < best_cost) {
+      best = nc;
+      best_cost = c;
+    }
+  }
+  return best;
 }
 
 // The decode-GEMV for batch 1 to 4, and for 5 to 16 when its items at the longest k-range
@@ -258,13 +275,24 @@ bool use_gemv(const trellis_desc* const* W, int count, int batch) {
   return items <= device_cus();
 }
 
-GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f16) {
+// Workspace bytes of a member's folded activations: rows of (x, x) pairs for 16 columns; above,
+// chunks of 32 rows of single values, which take no more than the rows of pairs from 16 rows on
+// (a plan's workspace must not grow past the no-allocation entry point's scratch; fewer rows
+// come here only where the column-block width is forced).
+size_t xf_bytes(int nc, int batch, int k) {
+  const size_t pairs = static_cast<size_t>(batch) * k * 4;
+  const size_t frags = static_cast<size_t>((batch + XF_CHUNK - 1) / XF_CHUNK) * (k / 16) * XF_FRAG;
+  return nc > 1 && frags > pairs ? frags : pairs;
+}
+
+// `split` off: the batched path's k-ranges are whole (no partial sums in the workspace).
+GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f16, bool split_k = true) {
   GroupPlan p;
   p.gemv = use_gemv(W, count, batch);
   p.nb = batch;
   p.nc = bgemm_nc(W, count, batch, f16);
   p.ncb = p.gemv ? 1 : (batch + 16 * p.nc - 1) / (16 * p.nc);
-  p.kr = p.gemv ? gemv_kr(W, count, batch) : bgemm_kr(W, count, batch, p.nc, f16);
+  p.kr = p.gemv ? gemv_kr(W, count, batch) : bgemm_kr(W, count, batch, p.nc, f16, split_k);
   // tiles per decode-GEMV stage: 16, or 8 for short k-ranges and for launches that split k
   // (a workgroup's first stage lands sooner: the 8B block's q/k/v and down launches
   // 0.2-0.7 us faster each at batch 1 to 8)
@@ -303,7 +331,7 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
       p.ws += align256(static_cast<size_t>(p.n_ob[i]) * p.ncb * p.S[i] * part_cols * 128 *
                        sizeof(float));
     p.off_xf[i] = p.ws;
-    if (!p.gemv) p.ws += align256(static_cast<size_t>(p.nb) * W[i]->k_in * 4);
+    if (!p.gemv) p.ws += align256(xf_bytes(p.nc, p.nb, W[i]->k_in));
   }
   return p;
 }
@@ -318,18 +346,25 @@ int launch_gemv(int K, int cb, int V, int kc, const LinArgs& g, hipStream_t st) 
   }
 }
 
-// The x fold of every member (the batched path), written once to the workspace.
-int launch_xfold(LinArgs& g, int folds, hipStream_t st) {
+// The x fold of every member (the batched path), written once to the workspace: in rows for
+// 16 batch columns, in MFMA fragments above.
+int launch_xfold(LinArgs& g, int nc, int folds, hipStream_t st) {
   const int items = g.total;
   g.total = folds;
-  const dim3 grid(static_cast<unsigned>((folds + 3) / 4));
   const bool one = g.nmat == 1;
-  if (xfold_rows(g.batch) == 4) {
-    if (one) hipLaunchKernelGGL((xfold_kernel<4, true>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((xfold_kernel<4, false>), grid, dim3(256), 0, st, g);
+  if (nc == 1) {
+    const dim3 grid(static_cast<unsigned>((folds + 3) / 4));
+    if (one) hipLaunchKernelGGL((xfold_kernel<true>), grid, dim3(256), 0, st, g);
+    else hipLaunchKernelGGL((xfold_kernel<false>), grid, dim3(256), 0, st, g);
   } else {
-    if (one) hipLaunchKernelGGL((xfold_kernel<1, true>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((xfold_kernel<1, false>), grid, dim3(256), 0, st, g);
+    const dim3 grid(static_cast<unsigned>(folds));
+    if (xfold_rows(nc, g.batch) == 32) {
+      if (one) hipLaunchKernelGGL((xfold_frag_kernel<4, true>), grid, dim3(512), 0, st, g);
+      else hipLaunchKernelGGL((xfold_frag_kernel<4, false>), grid, dim3(512), 0, st, g);
+    } else {
+      if (one) hipLaunchKernelGGL((xfold_frag_kernel<1, true>), grid, dim3(512), 0, st, g);
+      else hipLaunchKernelGGL((xfold_frag_kernel<1, false>), grid, dim3(512), 0, st, g);
+    }
   }
   g.total = items;
   return hipGetLastError() == hipSuccess ? TRELLIS_OK : TRELLIS_ERR_LAUNCH;
@@ -337,7 +372,7 @@ int launch_xfold(LinArgs& g, int folds, hipStream_t st) {
 
 // The batched path: the x fold, the decode-once batched kernel, and (split-K) its reduction.
 int launch_bgemm(int K, int cb, int V, int nc, LinArgs& g, int folds, int nfold, hipStream_t st) {
-  int v = launch_xfold(g, folds, st);
+  int v = launch_xfold(g, nc, folds, st);
   if (v) return v;
   switch (K) {
     case 2: v = launch_bgemm_k<2>(cb, V, nc, g, st); break;
@@ -621,8 +656,11 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
     if (static_cast<int64_t>(batch) * (batch > 1 ? ldx[i] : W[i]->k_in) * xes >= (int64_t(1) << 31))
       return TRELLIS_ERR_SHAPE;
   }
-  const GroupPlan p = group_plan(W, count, batch, f16);
+  GroupPlan p = group_plan(W, count, batch, f16);
   if (noalloc) {
+    // a batched plan whose partial sums do not fit the scratch goes without a split of k:
+    // what is left is the folded activations
+    if (p.ws > NOALLOC_SCRATCH_BYTES && !p.gemv) p = group_plan(W, count, batch, f16, false);
     if (p.ws > NOALLOC_SCRATCH_BYTES) return TRELLIS_ERR_SCRATCH;
     v = scratch_ptr(static_cast<hipStream_t>(stream), &workspace);
     if (v) return v;
@@ -652,6 +690,8 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
     m.osc = W[i]->osc;
     m.ldx = ldx[i];
     m.ldy = ldy[i];
+    m.y_words = y_dtype == TRELLIS_F32 ||
+                (reinterpret_cast<uintptr_t>(y[i]) % 4 == 0 && (batch == 1 || ldy[i] % 2 == 0));
     m.n = W[i]->n_out;
     m.k = W[i]->k_in;
     m.xfw = f16 ? ((W[i]->k_in + 31) / 32) * 16 : W[i]->k_in;
@@ -704,7 +744,7 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
       g.m[i].x = static_cast<const char*>(x[i]) + static_cast<size_t>(b0) * ldx[i] * xes;
       g.m[i].y = static_cast<char*>(y[i]) + static_cast<size_t>(b0) * ldy[i] * yes;
       g.m[i].chunk0 = chunk0;
-      chunk0 += ((g.batch + xfold_rows(g.batch) - 1) / xfold_rows(g.batch)) * ((W[i]->k_in + 127) / 128);
+      chunk0 += ((g.batch + xfold_rows(p.nc, g.batch) - 1) / xfold_rows(p.nc, g.batch)) * ((W[i]->k_in + 127) / 128);
     }
     v = p.gemv ? launch_gemv(W[0]->K, W[0]->codebook, W[0]->V, p.kc, g, st)
                : launch_bgemm(W[0]->K, W[0]->codebook, W[0]->V, p.nc, g, chunk0, nfold, st);
