@@ -44,6 +44,20 @@ def test_embed_rows_vs_oracle(te, gpu_device, n, k, cb, K, V):
     assert err.max() < TOL, err.max()
 
 
+@pytest.mark.parametrize("n,k", [(192, 192), (160, 96), (80, 320)])
+@pytest.mark.parametrize("K,cb", [(4, "mcg"), (2, "1mad")])
+def test_embed_rows_wave_shares(te, gpu_device, n, k, K, cb):
+    """Column blocks of 4, 2 and 4 tile columns (a wave takes one, or none) and row blocks of 4,
+    2 and 1 bands (fit 64, 32 and 16)."""
+    _say(f"[embed] wave shares n={n} k={k} K={K} cb={cb}")
+    bits, rec = tn.synthetic_record(n, k, K, seed=n * k, codebook=cb)
+    lin = make_linear(te, bits, rec, gpu_device)
+    W = tn.w_hat_from_record(bits, rec)
+    got = lin.embed_rows(torch.arange(n, dtype=torch.int32)).cpu().numpy().astype(np.float64)
+    err = np.abs(got - W).max(axis=1) / np.abs(W).max(axis=1)
+    assert err.max() < TOL, err.max()
+
+
 def test_embed_rows_out_of_range_and_f16(te, gpu_device):
     _say("[embed] ids out of range, f16 output, strided rows")
     bits, rec = tn.synthetic_record(256, 512, 3, seed=5)
