@@ -11,6 +11,8 @@
 #include <cstring>
 #include <mutex>
 
+#include <unistd.h>
+
 #include "trellis_amd.h"
 #include "decode.h"
 #define TRELLIS_XFOLD_DEFINE
@@ -83,9 +85,29 @@ int validate_fold(const trellis_desc* W) {
 }
 
 // ---------------------------------------------------------------- plan
-int env_int(const char* name, int dflt) {
-  const char* s = std::getenv(name);
-  return s ? std::atoi(s) : dflt;
+// The tuning knobs of the environment, read once per call in one pass over it (a getenv for
+// each knob walks the whole environment each time: together ~1 us of a call's host time).
+struct Knobs {
+  int gemv_kr = 0, gemv_kc = 0, bgemm_kr = 0, bgemm_nc = 0, small_batch_gemv = -1, plan_log = 0;
+};
+Knobs read_knobs() {
+  Knobs k;
+  if (!environ) return k;
+  for (char** e = environ; *e; ++e) {
+    if (std::strncmp(*e, "TRELLIS_", 8) != 0) continue;
+    const char* v = *e + 8;
+    auto take = [&](const char* name, int& to) {
+      const size_t n = std::strlen(name);
+      if (std::strncmp(v, name, n) == 0 && v[n] == '=') to = std::atoi(v + n + 1);
+    };
+    take("GEMV_KR", k.gemv_kr);
+    take("GEMV_KC", k.gemv_kc);
+    take("BGEMM_KR", k.bgemm_kr);
+    take("BGEMM_NC", k.bgemm_nc);
+    take("SMALL_BATCH_GEMV", k.small_batch_gemv);
+    take("PLAN_LOG", k.plan_log);
+  }
+  return k;
 }
 
 size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
@@ -132,12 +154,12 @@ int device_cus() {
 // activations of every row in each workgroup), plus ~2 us of split-K epilogue (publish,
 // ticket, reduce) and ~0.1 us of ticket contention per slice when kr does not cover k, plus
 // a first-load latency for every round after the first. TRELLIS_GEMV_KR forces a value.
-int gemv_kr(const trellis_desc* const* W, int count, int batch) {
+int gemv_kr(const trellis_desc* const* W, int count, int batch, const Knobs& kn) {
   const int nb = gemv_nb(batch), krm = gemv_kr_max(nb);
   int maxt = 0;
   for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
   const int cap = ((maxt + 7) / 8) * 8 < krm ? ((maxt + 7) / 8) * 8 : krm;
-  const int forced = env_int("TRELLIS_GEMV_KR", 0);
+  const int forced = kn.gemv_kr;
   if (forced >= 8 && forced <= krm && forced % 8 == 0) return forced;
   // the per-workgroup fold of every row (~2 model units per tile column and row)
   const long long per_kr = 100 + (nb > 4 ? 2 * nb : 0);
@@ -191,7 +213,7 @@ BgCost bgemm_cost(int nc, bool sum) {
 
 // Largest k-range with `split` off: one per block.
 int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool split,
-                  long long* cost) {
+                  const Knobs& kn, long long* cost) {
   int maxt = 0;
   for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
   const int kt = nc == 1 && !f16 ? 16 : 8;
@@ -199,7 +221,7 @@ int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bo
   const int cap = ((maxt + kt - 1) / kt) * kt;
   const long long cus = device_cus();
   const long long ncb = (batch + 16 * nc - 1) / (16 * nc);
-  const int forced = env_int("TRELLIS_BGEMM_KR", 0);
+  const int forced = kn.bgemm_kr;
   const bool force = split && forced >= kt && forced % kt == 0;
   int best = cap;
   long long best_cost = -1;
@@ -227,9 +249,10 @@ int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bo
   return best;
 }
 
-int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool split) {
+int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool split,
+             const Knobs& kn) {
   long long cost;
-  return bgemm_kr_cost(W, count, batch, nc, f16, split, &cost);
+  return bgemm_kr_cost(W, count, batch, nc, f16, split, kn, &cost);
 }
 
 // Column-block width in 16-column units: 1 up to 16 rows, 2 up to 32; above, the width that
@@ -237,8 +260,8 @@ int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f1
 // rows the 8B o launch takes 17.5 us in 32-column blocks and 19.7 in 64-column ones, gate+up
 // 53.7 and 40.8), else of 64, 128 and 256 (gate+up at 512 rows 246, 205 and 222 us, at 1024
 // rows 472, 395 and 365; o at 256 rows 33.0, 33.5 and 39.5).
-int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16) {
-  const int forced = env_int("TRELLIS_BGEMM_NC", 0);
+int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn) {
+  const int forced = kn.bgemm_nc;
   if (forced == 1 || forced == 2 || forced == 4 || forced == 8 || forced == 16) return forced;
   if (batch <= 16) return 1;
   if (batch <= 32) return 2;
@@ -246,7 +269,7 @@ int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16) {
   long long best_cost = 0;
   for (int nc = batch <= 64 ? 2 : 4; nc <= (batch <= 64 ? 4 : 16); nc *= 2) {
     long long c;
-    bgemm_kr_cost(W, count, batch, nc, f16, true, &c);
+    bgemm_kr_cost(W, count, batch, nc, f16, true, kn, &c);
     if (best == 0 || c < best_cost) {
       best = nc;
       best_cost = c;
@@ -263,10 +286,10 @@ int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16) {
 // q/k/v, o and down at batch 5 to 16, by 1-5 us per launch; gate+up needs two or more
 // rounds and loses by 4-15 us). TRELLIS_SMALL_BATCH_GEMV
 // = 1 / 0 forces the choice for batch 5 to 16.
-bool use_gemv(const trellis_desc* const* W, int count, int batch) {
+bool use_gemv(const trellis_desc* const* W, int count, int batch, const Knobs& kn) {
   if (batch <= 4) return true;
   if (batch > GEMV_MAX_NB) return false;
-  const int forced = env_int("TRELLIS_SMALL_BATCH_GEMV", -1);
+  const int forced = kn.small_batch_gemv;
   if (forced == 0 || forced == 1) return forced == 1;
   const int krm = gemv_kr_max(gemv_nb(batch));
   long long items = 0;
@@ -286,13 +309,14 @@ size_t xf_bytes(int nc, int batch, int k) {
 }
 
 // `split` off: the batched path's k-ranges are whole (no partial sums in the workspace).
-GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f16, bool split_k = true) {
+GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn,
+                     bool split_k = true) {
   GroupPlan p;
-  p.gemv = use_gemv(W, count, batch);
+  p.gemv = use_gemv(W, count, batch, kn);
   p.nb = batch;
-  p.nc = bgemm_nc(W, count, batch, f16);
+  p.nc = bgemm_nc(W, count, batch, f16, kn);
   p.ncb = p.gemv ? 1 : (batch + 16 * p.nc - 1) / (16 * p.nc);
-  p.kr = p.gemv ? gemv_kr(W, count, batch) : bgemm_kr(W, count, batch, p.nc, f16, split_k);
+  p.kr = p.gemv ? gemv_kr(W, count, batch, kn) : bgemm_kr(W, count, batch, p.nc, f16, split_k, kn);
   // tiles per decode-GEMV stage: 16, or 8 for short k-ranges and for launches that split k
   // (a workgroup's first stage lands sooner: the 8B block's q/k/v and down launches
   // 0.2-0.7 us faster each at batch 1 to 8)
@@ -300,7 +324,7 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
   for (int i = 0; i < count; ++i) split = split || W[i]->k_in / 16 > p.kr;
   p.kc = p.kr >= 32 && !(p.gemv && split) ? 16 : 8;
   {
-    const int kc = env_int("TRELLIS_GEMV_KC", 0);
+    const int kc = kn.gemv_kc;
     if (p.gemv && (kc == 8 || kc == 16) && kc <= p.kr) p.kc = kc;
   }
   // 16 rows: two 16-tile ring slots do not fit beside the rows' activations, so the
@@ -497,7 +521,8 @@ int trellis_workspace_bytes_group(const trellis_desc* const* W, int count, int b
   if (v) return v;
   if (batch < 1) return TRELLIS_ERR_BATCH;
   // either MFMA mode's plan fits (their k-ranges, hence partial buffers, may differ)
-  const size_t a = group_plan(W, count, batch, false).ws, b = group_plan(W, count, batch, true).ws;
+  const Knobs kn = read_knobs();
+  const size_t a = group_plan(W, count, batch, false, kn).ws, b = group_plan(W, count, batch, true, kn).ws;
   *bytes = a > b ? a : b;
   return TRELLIS_OK;
 }
@@ -638,8 +663,9 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
   int v = validate_group(W, count);
   if (v) return v;
   if (flags & ~TRELLIS_MMA_F16) return TRELLIS_ERR_FLAGS;
-  // the flag concerns the batched MFMA kernel only (the decode-GEMV is exact)
-  const bool f16 = (flags & TRELLIS_MMA_F16) != 0 && !use_gemv(W, count, batch);
+  const Knobs kn = read_knobs();
+  // the flag concerns the batched MFMA kernels only (the decode-GEMV is exact)
+  const bool f16 = (flags & TRELLIS_MMA_F16) != 0 && !use_gemv(W, count, batch, kn);
   if (!x || !y || !ldx || !ldy) return TRELLIS_ERR_NULL;
   if (batch < 1) return TRELLIS_ERR_BATCH;
   if ((x_dtype != TRELLIS_F32 && x_dtype != TRELLIS_F16) ||
@@ -656,11 +682,11 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
     if (static_cast<int64_t>(batch) * (batch > 1 ? ldx[i] : W[i]->k_in) * xes >= (int64_t(1) << 31))
       return TRELLIS_ERR_SHAPE;
   }
-  GroupPlan p = group_plan(W, count, batch, f16);
+  GroupPlan p = group_plan(W, count, batch, f16, kn);
   if (noalloc) {
     // a batched plan whose partial sums do not fit the scratch goes without a split of k:
     // what is left is the folded activations
-    if (p.ws > NOALLOC_SCRATCH_BYTES && !p.gemv) p = group_plan(W, count, batch, f16, false);
+    if (p.ws > NOALLOC_SCRATCH_BYTES && !p.gemv) p = group_plan(W, count, batch, f16, kn, false);
     if (p.ws > NOALLOC_SCRATCH_BYTES) return TRELLIS_ERR_SCRATCH;
     v = scratch_ptr(static_cast<hipStream_t>(stream), &workspace);
     if (v) return v;
@@ -719,7 +745,7 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
     g.m[i].fold0 = nfold;
     if (!p.gemv && p.S[i] > 1) nfold += p.n_ob[i] * p.ncb;
   }
-  if (env_int("TRELLIS_PLAN_LOG", 0))
+  if (kn.plan_log)
     std::fprintf(stderr, "trellis plan: batch=%d members=%d mode=%s kr=%d kc=%d nc=%d ncb=%d "
                          "items=%d S0=%d ws=%zu\n",
                  batch, count, p.gemv ? "gemv" : f16 ? "bgemm-f16" : "bgemm", p.kr, p.kc, p.nc,

@@ -51,8 +51,13 @@ class TrellisLinear(torch.nn.Module):
             y = x2.new_zeros((0, self.out_features), dtype=out_dtype)
         else:
             y = self.packed.forward(x2, out_dtype=out_dtype, mma_f16=self.mma_f16)
-        if self.bias is not None:
-            y = y + self.bias.to(y.dtype)
+        bias = self.bias
+        if bias is not None:
+            if x.dtype == torch.bfloat16 and not bias.requires_grad:
+                # the fp32 sum rounded once as it is stored: one kernel, not an add and a cast
+                y = torch.add(y, bias, out=torch.empty(y.shape, dtype=x.dtype, device=y.device))
+            else:
+                y = y + bias.to(y.dtype)
         return y.to(x.dtype).reshape(*lead, self.out_features)
 
     def extra_repr(self) -> str:

@@ -31,6 +31,10 @@ def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+# C dtype ids of the activation and output dtypes the kernels take
+_DT = {torch.float16: _capi.DT_F16, torch.float32: _capi.DT_F32}
+
+
 def _ws_size(need: int) -> int:
     """Bytes of a new workspace for `need`: the next power of two (at least 256), so a run
     of growing batch sizes replaces the buffer O(log n) times and the retired buffers
@@ -105,6 +109,7 @@ class PackedLinear:
             _ptr(self.bits), _ptr(self.su), _ptr(self.sv), _ptr(self.isc_scaled), _ptr(self.osc),
             self.n_out, self.k_in, self.K, self.V, _capi.CB_IDS[self.codebook],
             self.block_in, self.block_out, self.nwords)
+        self._desc_ref = ctypes.byref(self.desc)
         self._ws = None
         self._ws_retired = []
 
@@ -138,46 +143,50 @@ class PackedLinear:
         round each codebook value once to fp16 and use one MAC per weight in the batched
         kernel (TRELLIS_MMA_F16: ~2-3e-4 max rel err against the
         exact default, about half the MFMA work and activation traffic)."""
-        lib = _capi.load()
-        squeeze = x.dim() == 1
-        x2 = x.unsqueeze(0) if squeeze else x
-        if x2.dim() != 2 or x2.shape[1] != self.k_in:
-            raise ValueError(f"x shape {tuple(x.shape)} does not match k_in={self.k_in}")
-        if x2.device != self.device:
-            raise ValueError(f"x on {x2.device}, weights on {self.device}")
-        if x2.dtype not in (torch.float16, torch.float32):
-            raise ValueError(f"x dtype {x2.dtype} not supported")
-        if x2.stride(1) != 1:
-            x2 = x2.contiguous()
-        B = x2.shape[0]
+        # (attribute reads and small objects are most of an eager call's host time: each is
+        # taken once, and nothing is built that the call does not need)
+        fn = _capi.load().trellis_packed_linear_ex
+        shape, squeeze = x.shape, x.dim() == 1
+        if len(shape) not in (1, 2) or shape[-1] != self.k_in:
+            raise ValueError(f"x shape {tuple(shape if not squeeze else (1, *shape))} does not match "
+                             f"k_in={self.k_in}")
+        dev = self.device
+        if x.device != dev:
+            raise ValueError(f"x on {x.device}, weights on {dev}")
+        xdt = _DT.get(x.dtype)
+        if xdt is None:
+            raise ValueError(f"x dtype {x.dtype} not supported")
+        if x.stride(-1) != 1:
+            x = x.contiguous()
+        B, ldx = (1, self.k_in) if squeeze else (shape[0], x.stride(0))
         if out is None:
-            out = torch.empty((B, self.n_out), dtype=out_dtype, device=self.device)
-        y2 = out.view(B, self.n_out) if out.dim() == 1 else out
-        if y2.dtype not in (torch.float16, torch.float32) or y2.stride(1) != 1:
+            # one allocation of the returned shape
+            y = torch.empty(self.n_out if squeeze else (B, self.n_out), dtype=out_dtype, device=dev)
+            ydt, ldy, ret = _DT.get(out_dtype), self.n_out, y
+        else:
+            y = out.view(B, self.n_out) if out.dim() == 1 else out
+            ydt, ldy = _DT.get(y.dtype) if y.stride(1) == 1 else None, y.stride(0)
+            ret = out[0] if (squeeze and out.dim() == 2) else out
+        if ydt is None:
             raise ValueError("out must be fp16/fp32 with unit column stride")
         if B == 0:
             # no rows, nothing to launch (the C ABI rejects a batch of 0)
-            return out
-        stream = ctypes.c_void_p(_stream(self.device))
-        xdt = _capi.DT_F16 if x2.dtype == torch.float16 else _capi.DT_F32
-        ydt = _capi.DT_F16 if y2.dtype == torch.float16 else _capi.DT_F32
+            return out if out is not None else y
         flags = _capi.MMA_F16 if mma_f16 else 0
-
-        def launch(ws):
-            return lib.trellis_packed_linear_ex(
-                ctypes.byref(self.desc), _ptr(x2), x2.stride(0), B, xdt, _ptr(y2), y2.stride(0),
-                ydt, _ptr(ws), ws.numel(), flags, stream)
-
-        if workspace is not None:
-            st = launch(workspace)
-        else:
-            # the library checks the workspace size before it launches anything, so the
-            # current buffer is tried first and sized (grown) only when it is too small
-            st = launch(self._ws) if self._ws is not None else _capi.ERR_WORKSPACE
-            if st == _capi.ERR_WORKSPACE:
-                st = launch(self._workspace(B))
-        _capi.check(st)
-        return out[0] if (squeeze and out.dim() == 2) else out
+        stream = _stream(dev)
+        # the library checks the workspace size before it launches anything, so the current
+        # buffer is tried first and sized (grown) only when it is too small
+        ws = workspace if workspace is not None else self._ws
+        st = _capi.ERR_WORKSPACE if ws is None else fn(
+            self._desc_ref, x.data_ptr(), ldx, B, xdt, y.data_ptr(), ldy, ydt, ws.data_ptr(),
+            ws.numel(), flags, stream)
+        if st == _capi.ERR_WORKSPACE and workspace is None:
+            ws = self._workspace(B)
+            st = fn(self._desc_ref, x.data_ptr(), ldx, B, xdt, y.data_ptr(), ldy, ydt,
+                    ws.data_ptr(), ws.numel(), flags, stream)
+        if st:
+            _capi.check(st)
+        return ret
 
     __call__ = forward
 
@@ -236,6 +245,8 @@ class PackedGroup:
         self._descs = (_capi.TrellisDesc * n)(*[lin.desc for lin in linears])
         self._dptrs = (ctypes.POINTER(_capi.TrellisDesc) * n)(
             *[ctypes.pointer(self._descs[i]) for i in range(n)])
+        self._ptrs, self._strides = ctypes.c_void_p * n, ctypes.c_int64 * n
+        self._n_outs = [lin.n_out for lin in linears]
         self._ws = None
         self._ws_retired = []
 
@@ -257,51 +268,58 @@ class PackedGroup:
                 mma_f16: bool = False):
         """xs: one activation per member ([k_i] or [batch, k_i], same batch and dtype);
         returns (or fills) one output per member. mma_f16 as PackedLinear.forward."""
-        lib = _capi.load()
-        n = len(self.linears)
+        fn = _capi.load().trellis_packed_linear_group_ex
+        lins = self.linears
+        n = len(lins)
         if len(xs) != n:
             raise ValueError(f"expected {n} inputs")
+        dev, dt = self.device, xs[0].dtype
         squeeze = xs[0].dim() == 1
-        x2 = [x.unsqueeze(0) if x.dim() == 1 else x for x in xs]
-        x2 = [x if x.stride(1) == 1 else x.contiguous() for x in x2]
-        B = x2[0].shape[0]
-        dt = x2[0].dtype
-        for lin, x in zip(self.linears, x2):
-            if x.shape != (B, lin.k_in) or x.dtype != dt or x.device != self.device:
+        B = 1 if squeeze else xs[0].shape[0]
+        x2, ldx = [], []
+        for lin, x in zip(lins, xs):
+            one = x.dim() == 1
+            if ((1, *x.shape) if one else tuple(x.shape)) != (B, lin.k_in) or x.dtype != dt or x.device != dev:
                 raise ValueError("inputs must share batch, dtype and device and match k_in")
-        if dt not in (torch.float16, torch.float32):
+            if x.stride(-1) != 1:
+                x = x.contiguous()
+            x2.append(x)
+            ldx.append(lin.k_in if one else x.stride(0))
+        xdt = _DT.get(dt)
+        if xdt is None:
             raise ValueError(f"x dtype {dt} not supported")
         if outs is None:
-            outs = [torch.empty((B, lin.n_out), dtype=out_dtype, device=self.device)
-                    for lin in self.linears]
-        y2 = [o.view(B, lin.n_out) if o.dim() == 1 else o for o, lin in zip(outs, self.linears)]
-        ydt = y2[0].dtype
-        if any(y.dtype != ydt or y.stride(1) != 1 for y in y2) or ydt not in (torch.float16,
-                                                                               torch.float32):
+            y2 = [torch.empty(lin.n_out if squeeze else (B, lin.n_out), dtype=out_dtype, device=dev)
+                  for lin in lins]
+            ret, ydt, ldy = y2, _DT.get(out_dtype), self._n_outs
+        else:
+            y2 = [o.view(B, lin.n_out) if o.dim() == 1 else o for o, lin in zip(outs, lins)]
+            ydt = _DT.get(y2[0].dtype)
+            if any(y.dtype != y2[0].dtype or y.stride(1) != 1 for y in y2):
+                ydt = None
+            ldy = [y.stride(0) for y in y2]
+            ret = [o[0] if o.dim() == 2 else o for o in outs] if squeeze else outs
+        if ydt is None:
             raise ValueError("outputs must share an fp16/fp32 dtype with unit column stride")
         if B == 0:
             # no rows: every member's output is [0, n_i], nothing to launch
-            return outs
-        xp = (ctypes.c_void_p * n)(*[x.data_ptr() for x in x2])
-        yp = (ctypes.c_void_p * n)(*[y.data_ptr() for y in y2])
-        ldx = (ctypes.c_int64 * n)(*[x.stride(0) for x in x2])
-        ldy = (ctypes.c_int64 * n)(*[y.stride(0) for y in y2])
-        stream = ctypes.c_void_p(_stream(self.device))
-
-        def launch(ws):
-            return lib.trellis_packed_linear_group_ex(
-                self._dptrs, n, xp, ldx, B, _capi.DT_F16 if dt == torch.float16 else _capi.DT_F32,
-                yp, ldy, _capi.DT_F16 if ydt == torch.float16 else _capi.DT_F32,
-                _ptr(ws), ws.numel(), _capi.MMA_F16 if mma_f16 else 0, stream)
-
+            return outs if outs is not None else y2
+        xp = self._ptrs(*[x.data_ptr() for x in x2])
+        yp = self._ptrs(*[y.data_ptr() for y in y2])
+        lx, ly = self._strides(*ldx), self._strides(*ldy)
+        flags = _capi.MMA_F16 if mma_f16 else 0
+        stream = _stream(dev)
         # as PackedLinear.forward: the current workspace first, sized only when too small
-        st = launch(self._ws) if self._ws is not None else _capi.ERR_WORKSPACE
+        ws = self._ws
+        st = _capi.ERR_WORKSPACE if ws is None else fn(
+            self._dptrs, n, xp, lx, B, xdt, yp, ly, ydt, ws.data_ptr(), ws.numel(), flags, stream)
         if st == _capi.ERR_WORKSPACE:
-            st = launch(self._workspace(B))
-        _capi.check(st)
-        if squeeze:
-            return [o[0] if o.dim() == 2 else o for o in outs]
-        return outs
+            ws = self._workspace(B)
+            st = fn(self._dptrs, n, xp, lx, B, xdt, yp, ly, ydt, ws.data_ptr(), ws.numel(), flags,
+                    stream)
+        if st:
+            _capi.check(st)
+        return ret
 
     __call__ = forward
 
