@@ -43,3 +43,22 @@ def test_widths_at_tile_edges(te, gpu_device, monkeypatch, nc, n, k, K, cb, V, b
             assert tn.rel_err(buf[:, 1:1 + n].float().cpu().numpy(), want) < TOL + 2.0 ** -11, (f16, kr)
             pad = torch.cat([buf[:, :1], buf[:, 1 + n:]], 1)
             assert torch.equal(pad, torch.full_like(pad, 7.0)), (f16, kr)
+
+
+@pytest.mark.parametrize("n,k,K,cb,V,batch,f16", [
+    (144, 48, 3, "mcg", 1, 17, True), (272, 336, 2, "3inst", 2, 33, True), (128, 2064, 4, "1mad", 1, 65, True),
+    (400, 1040, 3, "mcg", 1, 129, True), (96, 8192, 3, "mcg", 1, 64, True), (144, 528, 4, "mcg", 2, 257, True),
+    (272, 8192, 3, "mcg", 1, 17, False), (128, 8208, 2, "3inst", 2, 64, False)])
+def test_shared_activation_kernel(te, gpu_device, n, k, K, cb, V, batch, f16):
+    """The 16-wave kernel above 16 rows, as the planner picks it (fp16-weight mode, and the
+    exact mode with a k of 8192 and more), split k and odd tiles included."""
+    print(f"[shared] n={n} k={k} K={K} cb={cb} V={V} batch={batch} f16={f16}", flush=True)
+    bits, rec = tn.synthetic_record(n, k, K, seed=n + k, codebook=cb, V=V)
+    lin = te.PackedLinear(te.PackedRecord(rec.n, rec.k, rec.K, bits, rec.su, rec.sv, rec.isc, rec.osc,
+                                          float(rec.scale), codebook=rec.codebook, V=rec.V),
+                          device=gpu_device)
+    x = np.random.default_rng(batch).standard_normal((batch, k)).astype(np.float16)
+    xt = torch.from_numpy(x).to(gpu_device)
+    y = lin(xt, mma_f16=f16)
+    assert tn.rel_err(y.cpu().numpy(), tn.packed_linear_ref(bits, rec, x)) < TOL
+    assert torch.equal(y, lin(xt, mma_f16=f16))

@@ -1,7 +1,8 @@
 // bgemm.h — batched packed linear for gfx950: decode once, reuse across the batch. Three
 // kernels by the call's rows, each a 128-row output block (the out-dim Hadamard block) x a
 // block of batch columns x one k-range per workgroup, one workgroup per CU:
-//   bgemm16_kernel    up to 16 rows: 16 waves, activations shared through LDS;
+//   bgemm_shared_kernel 16 waves, activations shared through LDS: up to 16 rows, and above
+//                     where the planner's rule finds it faster (bgemm_shared);
 //   bgemm_kernel      32 or 64 columns: 8 waves, each with its own share of the k-range;
 //   bgemm_wide_kernel 128 or 256 columns: 4 waves with 64 accumulator tiles each.
 // In each a wave decodes a tile once, straight into the A operand of an MFMA (common.h), and
@@ -85,6 +86,14 @@ __device__ __forceinline__ void bg_out_fold(const LinArgs& g, const LinMat& m, c
 
 constexpr int BG_LDS_WORDS = 160 * 1024 / 4;
 
+// LDS regions of bgemm_shared_kernel's epilogue sums, at most one per k-lane.
+__host__ __device__ constexpr int bg_regions(int nb, int kl, int tls, int xbuf, int other) {
+  const int limit = nb < 64 ? BG_LDS_WORDS / 2 : BG_LDS_WORDS, base = 2 * xbuf;
+  int r = kl;
+  while (r > 1 && (r * nb * tls > base ? r * nb * tls : base) + other > limit) r /= 2;
+  return r;
+}
+
 // s_setprio with a value known after unrolling (the instruction takes an immediate)
 __device__ __forceinline__ void setprio_n(int v) {
   if (v >= 3) __builtin_amdgcn_s_setprio(3);
@@ -93,7 +102,7 @@ __device__ __forceinline__ void setprio_n(int v) {
   else __builtin_amdgcn_s_setprio(0);
 }
 
-// ---------------------------------------------------------------- up to 16 columns
+// ---------------------------------------------------------------- shared activations
 // A workgroup of 16 waves: wave w = (band group bg = w % NG, k-lane kl = w / NG), a band group
 // being BW adjacent bands; the waves of a SIMD share a band group and split every k-step's
 // tiles between them (tile j of a step belongs to k-lane j % KL):
@@ -107,19 +116,20 @@ __device__ __forceinline__ void setprio_n(int v) {
 //     matrix read zeros), so none is clamped or skipped and the waits stay exact;
 //   * the B rows are padded by 8 words (a row stride of 8 mod 64 words: the fragments' reads
 //     spread over the banks);
-//   * the epilogue adds the k-lanes' sums into t[16][128] in LDS in k-lane order.
-// At 16 rows the kernels for more columns measured slower (8B gate+up 28.9 us with 32-column
+//   * the epilogue adds the k-lanes' sums into t[16 NC][128] in LDS in k-lane order.
+// At 16 rows the kernels below measured slower (8B gate+up 28.9 us with 32-column
 // blocks, 26.5 with this one; q/k/v 16.5 and 15.9, o 14.7 and 13.2, down 19.5 and 17.3).
-template <int K, int CB, int V, int F16, bool SINGLE>
-__global__ __launch_bounds__(1024) void bgemm16_kernel(LinArgs g) {
-  constexpr int NC = 1, BG_WAVES = 16;
+template <int K, int CB, int V, int NC, int F16, bool SINGLE>
+__global__ __launch_bounds__(1024) void bgemm_shared_kernel(LinArgs g) {
+  constexpr int BG_WAVES = 16;
+  static_assert(F16 || NC <= 4, "exact mode: up to 64 columns");
   constexpr int NWK = 8 * K;
-  // tile columns per k-step: 16 (half the barriers of 8; the 8B gate+up group 29.1 -> 27.9 us),
-  // 8 in the fp16-weight mode, a pair per k-lane
-  constexpr int KT = F16 ? 8 : 16;
-  // bands per wave: 4 (8 k-lanes; each B fragment read from LDS feeds 4 bands: 27.8 ->
-  // 26.6-27.1 us), 2 in the fp16-weight mode
-  constexpr int BW = F16 ? 2 : 4;
+  // tile columns per k-step: at 16 columns 16 (half the barriers of 8; the 8B gate+up group 29.1 -> 27.9 us),
+  // otherwise 8 (in the fp16-weight mode a pair per k-lane)
+  constexpr int KT = F16 || NC > 1 ? 8 : 16;
+  // bands per wave: at 16 columns 4 (8 k-lanes; each B fragment read from LDS feeds 4 bands: 27.8 ->
+  // 26.6-27.1 us), otherwise 2
+  constexpr int BW = F16 || NC > 1 ? 2 : 4;
   constexpr int NG = 8 / BW;                       // band groups of the block
   constexpr int KL = BG_WAVES / NG;                // k-lanes: waves of one band group
   // tiles per band per k-lane per step: exact mode, tiles kl, kl + KL, ...; fp16-weight
@@ -128,7 +138,7 @@ __global__ __launch_bounds__(1024) void bgemm16_kernel(LinArgs g) {
   static_assert(F16 || (KT % KL == 0 && TPL >= 1), "a tile column per k-lane per step");
   constexpr int WPT = F16 ? 8 : 16;                // B words per tile column and batch row
   constexpr int XW = KT * WPT + 8;                 // LDS words per B row (+8: bank spread)
-  constexpr int NB = 16;                           // batch columns per workgroup
+  constexpr int NB = 16 * NC;                      // batch columns per workgroup
   constexpr int RCH = KT * WPT / 4;                // 16-byte chunks per B row per step
   constexpr int XCH = NB * RCH;                    // 16-byte B chunks per step
   constexpr int XLOADS = (XCH + 64 * BG_WAVES - 1) / (64 * BG_WAVES);
@@ -140,13 +150,13 @@ __global__ __launch_bounds__(1024) void bgemm16_kernel(LinArgs g) {
   static_assert(!F16 || (KT == 2 * KL && BW == 2), "fp16-weight mode: one tile pair per k-lane per step");
   // epilogue: t[NB][TLS] (rows padded like the B rows, so a fragment's float4 writes spread
   // over the banks) in NR regions NR_OFF floats apart over the B buffers (k-lanes
-  // k2 .. k2 + NR - 1 add into regions 0 .. NR - 1 in round k2 / NR). Four regions: more
-  // would leave no room for two workgroups per CU (against two: 26.1 -> 25.9 us)
+  // k2 .. k2 + NR - 1 add into regions 0 .. NR - 1 in round k2 / NR). As many as
+  // the LDS holds, below 64 columns half of it: two workgroups fit a CU (bg_regions)
   constexpr int TLS = 136;
-  constexpr int NR = 4;
+  constexpr int NR = bg_regions(NB, KL, TLS, XBUF, BG_WAVES * BSW);
   constexpr int NR_OFF = NB * TLS;
   constexpr int XSB = 2 * XBUF > NR * NR_OFF ? 2 * XBUF : NR * NR_OFF;
-  static_assert(KL % NR == 0 && XSB + BG_WAVES * BSW <= BG_LDS_WORDS / 2, "epilogue regions");
+  static_assert(KL % NR == 0 && NB * TLS <= XSB && XSB + BG_WAVES * BSW <= BG_LDS_WORDS, "epilogue regions");
   __shared__ __align__(16) uint32_t xsb[XSB];
   __shared__ __align__(16) uint32_t bst[BG_WAVES * BSW];
   float* tl = reinterpret_cast<float*>(xsb);

@@ -394,11 +394,13 @@ __device__ __forceinline__ int xf_pair_slot(int e) {
 // v_mfma_f32_32x32x16_f16, lane l = (row l % 32, h = l / 32), read as one coalesced load.
 constexpr int XF_CHUNK = 32;          // batch rows per chunk
 constexpr int XF_FRAG = 1024;         // bytes per (chunk, tile column)
-// batch rows per x-fold job: one for the 16-row kernel's layout; above, a workgroup's 8, or 32
+// batch rows per x-fold job: a wave's one, or four, in the row layout; in fragments a workgroup's 8, or 32
 // (four per wave, their scales loaded once and the rows transformed together) from 256 rows
 // up, where a launch needs several rounds of waves on the CUs, each paying the start-up latency
 // (8B block at 512 rows 517 -> 503.5 us; at 128 rows no change)
-__host__ __device__ constexpr int xfold_rows(int nc, int batch) { return nc == 1 ? 1 : batch >= 256 ? 32 : 8; }
+__host__ __device__ constexpr int xfold_rows(bool frag, int batch) {
+  return frag ? (batch >= 256 ? 32 : 8) : (batch >= 256 ? 4 : 1);
+}
 #ifdef TRELLIS_XFOLD_DEFINE
 // The x fold into that layout. One wave per R batch rows (8 apart) of a group of 8 R, all of
 // one 128-column chunk, so a workgroup of 8 waves holds runs of 8 R rows of each 16-byte
@@ -473,7 +475,7 @@ __global__ __launch_bounds__(512) void xfold_frag_kernel(LinArgs g) {
 // chunk), every load a range-checked buffer load issued up front: a few rows are latency-
 // bound, and one row per wave gives every SIMD several waves to overlap the transform's
 // dependent lane exchanges.
-template <bool SINGLE>
+template <int XFOLD_ROWS, bool SINGLE>
 __global__ __launch_bounds__(256) void xfold_kernel(LinArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int job = blockIdx.x * 4 + wave;
@@ -483,7 +485,8 @@ __global__ __launch_bounds__(256) void xfold_kernel(LinArgs g) {
   const LinMat& m = g.m[mi];
   const int local = job - m.chunk0;
   const int nch = (m.k + 127) / 128;
-  const int b0 = local / nch, ch = local % nch;
+  const int rg = local / nch, ch = local % nch;
+  const int b0 = rg * XFOLD_ROWS;
   const int kvalid = min(128, m.k - ch * 128);
   const int xsh = g.x_f16 ? 1 : 2;
   const rsrc_t r_x = make_rsrc(m.x, static_cast<unsigned>(g.batch) * static_cast<unsigned>(m.ldx) << xsh);
@@ -493,24 +496,41 @@ __global__ __launch_bounds__(256) void xfold_kernel(LinArgs g) {
                    __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_isc, e0 * 4, 0, 0));
   const float s1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_su, e1 * 4, 0, 0)) *
                    __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_isc, e1 * 4, 0, 0));
-  const unsigned row = static_cast<unsigned>(b0 * m.ldx);
-  const uint32_t w0 = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e0) << xsh) & ~3u), 0, 0);
-  const uint32_t w1 = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e1) << xsh) & ~3u), 0, 0);
+  uint32_t w0[XFOLD_ROWS], w1[XFOLD_ROWS];
+#pragma unroll
+  for (int r = 0; r < XFOLD_ROWS; ++r) {
+    const unsigned row = static_cast<unsigned>((b0 + r) * m.ldx);
+    w0[r] = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e0) << xsh) & ~3u), 0, 0);
+    w1[r] = __builtin_amdgcn_raw_buffer_load_b32(r_x, static_cast<int>(((row + e1) << xsh) & ~3u), 0, 0);
+  }
   const float nrm = m.nrm_in;
-  // an f16 row stride is even, so the element's half within its word follows e
-  float lo = lane < kvalid ? act_value(w0, e0, g.x_f16) * s0 : 0.0f;
-  float hi = lane + 64 < kvalid ? act_value(w1, e1, g.x_f16) * s1 : 0.0f;
-  fwht_chunk(lo, hi, m.block_in, lane);
-  if (g.mma_f16) {
-    // columns k .. kp - 1 of the last pair are written as zeros (lo and hi are zero there)
-    _Float16* dst = reinterpret_cast<_Float16*>(m.xf + static_cast<size_t>(b0) * m.xfw);
-    const int kp = 2 * m.xfw;
-    if (e0 < kp) st_wt(dst + xf_pair_slot(e0), static_cast<_Float16>(lo * nrm));
-    if (e1 < kp) st_wt(dst + xf_pair_slot(e1), static_cast<_Float16>(hi * nrm));
-  } else {
-    uint32_t* dst = m.xf + static_cast<size_t>(b0) * m.xfw + ch * 128;
-    if (lane < kvalid) st_wt(dst + lane, dup_half(lo * nrm));
-    if (lane + 64 < kvalid) st_wt(dst + lane + 64, dup_half(hi * nrm));
+  const FwhtLane fl = fwht_lane(lane, m.block_in);
+  // the rows are transformed together, level by level, so their dependent lane exchanges
+  // overlap (rows past the call's were loaded as zeros and are not stored)
+  float lov[XFOLD_ROWS], hiv[XFOLD_ROWS];
+#pragma unroll
+  for (int r = 0; r < XFOLD_ROWS; ++r) {
+    // an f16 row stride is even, so the element's half within its word follows e
+    lov[r] = lane < kvalid ? act_value(w0[r], e0, g.x_f16) * s0 : 0.0f;
+    hiv[r] = lane + 64 < kvalid ? act_value(w1[r], e1, g.x_f16) * s1 : 0.0f;
+  }
+  fwht_chunks<XFOLD_ROWS>(lov, hiv, m.block_in, lane, fl);
+#pragma unroll
+  for (int r = 0; r < XFOLD_ROWS; ++r) {
+    if (b0 + r >= g.batch) break;
+    const float lo = lov[r], hi = hiv[r];
+    if (g.mma_f16) {
+      // fp16 values in tile-pair order (xf_pair_slot); columns k .. kp - 1 of the last
+      // pair are written as zeros (lo and hi are zero there)
+      _Float16* dst = reinterpret_cast<_Float16*>(m.xf + static_cast<size_t>(b0 + r) * m.xfw);
+      const int kp = 2 * m.xfw;
+      if (e0 < kp) st_wt(dst + xf_pair_slot(e0), static_cast<_Float16>(lo * nrm));
+      if (e1 < kp) st_wt(dst + xf_pair_slot(e1), static_cast<_Float16>(hi * nrm));
+    } else {
+      uint32_t* dst = m.xf + static_cast<size_t>(b0 + r) * m.xfw + ch * 128;
+      if (lane < kvalid) st_wt(dst + lane, dup_half(lo * nrm));
+      if (lane + 64 < kvalid) st_wt(dst + lane + 64, dup_half(hi * nrm));
+    }
   }
 }
 #endif

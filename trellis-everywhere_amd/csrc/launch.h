@@ -19,10 +19,10 @@ constexpr int gemv_nb(int batch) { return batch <= 1 ? 1 : batch == 2 ? 2 : batc
 template <int K>
 int launch_gemv_k(int cb, int V, int kc, const LinArgs& g, hipStream_t st);
 
-// The batched kernel for column blocks of 16 nc (bgemm16_kernel, bgemm_kernel,
+// The batched kernel for column blocks of 16 nc (bgemm_shared_kernel, bgemm_kernel,
 // bgemm_wide_kernel) over g.total items (the x fold has been launched before it).
 template <int K>
-int launch_bgemm_k(int cb, int V, int nc, const LinArgs& g, hipStream_t st);
+int launch_bgemm_k(int cb, int V, int nc, bool shared, const LinArgs& g, hipStream_t st);
 
 // bfold_kernel<cb, nc> over nfold (block, column block) jobs of 4 * nc workgroups each
 // (after a split-K bgemm_kernel).
@@ -110,7 +110,7 @@ int launch_gemv_k(int cb, int V, int kc, const LinArgs& g, hipStream_t st) {
 }
 
 template <int K, int CB, int V, int F16>
-static int launch_bgemm_nc(int nc, const LinArgs& g, hipStream_t st) {
+static int launch_bgemm_nc(int nc, bool shared, const LinArgs& g, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(g.total));
   const bool one = g.nmat == 1;
   // 1MAD's values are exact in one fp16: above 16 columns its exact mode is the fp16-weight one
@@ -118,8 +118,18 @@ static int launch_bgemm_nc(int nc, const LinArgs& g, hipStream_t st) {
 #define TRELLIS_BG_LAUNCH(KERNEL, THREADS, ...) \
   if (one) hipLaunchKernelGGL((KERNEL<K, CB, V, __VA_ARGS__, true>), grid, dim3(THREADS), 0, st, g); \
   else hipLaunchKernelGGL((KERNEL<K, CB, V, __VA_ARGS__, false>), grid, dim3(THREADS), 0, st, g);
+  if (shared) {
+    switch (nc) {
+      case 1: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 1, F16) break;
+      case 2: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 2, F16) break;
+      case 4: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 4, F16) break;
+      default:
+        if constexpr (F16) { TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 8, F16) }
+        else return 13;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : 13;
+  }
   switch (nc) {
-    case 1: TRELLIS_BG_LAUNCH(bgemm16_kernel, 1024, F16) break;
     case 2: TRELLIS_BG_LAUNCH(bgemm_kernel, 512, 2, F) break;
     case 4: TRELLIS_BG_LAUNCH(bgemm_kernel, 512, 4, F) break;
     case 8: TRELLIS_BG_LAUNCH(bgemm_wide_kernel, 256, 8, F) break;
@@ -130,21 +140,21 @@ static int launch_bgemm_nc(int nc, const LinArgs& g, hipStream_t st) {
 }
 
 template <int K, int CB, int V>
-static int launch_bgemm_f(int nc, const LinArgs& g, hipStream_t st) {
-  return g.mma_f16 ? launch_bgemm_nc<K, CB, V, 1>(nc, g, st) : launch_bgemm_nc<K, CB, V, 0>(nc, g, st);
+static int launch_bgemm_f(int nc, bool shared, const LinArgs& g, hipStream_t st) {
+  return g.mma_f16 ? launch_bgemm_nc<K, CB, V, 1>(nc, shared, g, st) : launch_bgemm_nc<K, CB, V, 0>(nc, shared, g, st);
 }
 
 template <int K, int CB>
-static int launch_bgemm_v(int V, int nc, const LinArgs& g, hipStream_t st) {
-  return V == 2 ? launch_bgemm_f<K, CB, 2>(nc, g, st) : launch_bgemm_f<K, CB, 1>(nc, g, st);
+static int launch_bgemm_v(int V, int nc, bool shared, const LinArgs& g, hipStream_t st) {
+  return V == 2 ? launch_bgemm_f<K, CB, 2>(nc, shared, g, st) : launch_bgemm_f<K, CB, 1>(nc, shared, g, st);
 }
 
 template <int K>
-int launch_bgemm_k(int cb, int V, int nc, const LinArgs& g, hipStream_t st) {
+int launch_bgemm_k(int cb, int V, int nc, bool shared, const LinArgs& g, hipStream_t st) {
   switch (cb) {
-    case CB_MCG: return launch_bgemm_v<K, CB_MCG>(V, nc, g, st);
-    case CB_3INST: return launch_bgemm_v<K, CB_3INST>(V, nc, g, st);
-    default: return launch_bgemm_v<K, CB_1MAD>(V, nc, g, st);
+    case CB_MCG: return launch_bgemm_v<K, CB_MCG>(V, nc, shared, g, st);
+    case CB_3INST: return launch_bgemm_v<K, CB_3INST>(V, nc, shared, g, st);
+    default: return launch_bgemm_v<K, CB_1MAD>(V, nc, shared, g, st);
   }
 }
 #endif

@@ -116,6 +116,7 @@ struct GroupPlan {
   int nb;              // batch rows per launch
   int gemv;            // batch-1 gemv_kernel (else bgemm_kernel)
   int nc, ncb;         // bgemm: 16-column chunks per workgroup, column blocks
+  bool shared;         // bgemm_shared_kernel
   int kr;              // gemv / bgemm: tile columns per k-range
   int kc;              // gemv: tile columns per pipeline stage (8 or 16)
   int total;           // work items over the group
@@ -212,12 +213,15 @@ BgCost bgemm_cost(int nc, bool sum) {
 }
 
 // Largest k-range with `split` off: one per block.
-int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool split,
-                  const Knobs& kn, long long* cost) {
+int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool shared,
+                  bool split, const Knobs& kn, long long* cost) {
   int maxt = 0;
   for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
   const int kt = nc == 1 && !f16 ? 16 : 8;
-  const BgCost bc = bgemm_cost(nc, f16 || W[0]->codebook == TRELLIS_CB_1MAD);
+  // (bgemm_shared_kernel above 16 rows: its step costs and launch terms, in ns at 2.4 GHz)
+  const bool row = shared && nc > 1;
+  const BgCost bc = row ? BgCost{(f16 ? 75 + 10 * nc : 61 + 19 * nc) * 10 / 24, 1500}
+                        : bgemm_cost(nc, f16 || W[0]->codebook == TRELLIS_CB_1MAD);
   const int cap = ((maxt + kt - 1) / kt) * kt;
   const long long cus = device_cus();
   const long long ncb = (batch + 16 * nc - 1) / (16 * nc);
@@ -238,7 +242,7 @@ int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bo
     if (smax > 16 && !force) continue;
     const long long rounds = (items + cus - 1) / cus;
     const long long c = rounds * (2LL * kr * bc.tile + bc.item) +
-                        (smax > 1 ? 3500 + part_bytes / 4500 : 0);
+                        (smax > 1 ? (row ? 1500 + part_bytes / 3000 : 3500 + part_bytes / 4500) : 0);
     if (best_cost < 0 || c < best_cost) {
       best = kr;
       best_cost = c;
@@ -249,10 +253,30 @@ int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bo
   return best;
 }
 
-int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool split,
-             const Knobs& kn) {
+int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool shared,
+             bool split, const Knobs& kn) {
   long long cost;
-  return bgemm_kr_cost(W, count, batch, nc, f16, split, kn, &cost);
+  return bgemm_kr_cost(W, count, batch, nc, f16, shared, split, kn, &cost);
+}
+
+// Which batched kernel above 16 rows: bgemm_shared_kernel (16 waves, B shared through LDS), or
+// the streaming ones. With weights that come from HBM (a model's, 14 copies of the 8B block in
+// turn, K=3 MCG) the shared one's four waves per SIMD hide more of the loads' latency, and the
+// streaming ones have cheaper products:
+//   exact, up to 64 rows, long k that is split: down (768 tile columns) at 32 / 64 rows shared
+//   20.2 / 26.6 us, streaming 20.9 / 29.4; shorter k at 64 rows q/k/v 22.3 and 21.8, o 16.9 and
+//   16.7, gate+up 41.3 and 40.9 (34.7 with its weights in the last-level cache).
+//   fp16-weight mode, up to 64 rows: block at 32 / 64 rows shared 77.9 / 97.5, streaming 83.5 /
+//   103.1. At 128 / 512 rows, k of 4096: gate+up 47.0 / 154.7 and 54.6 / 162.5, q/k/v 26.7 /
+//   52.2 and 27.8 / 58.6; long k: down 32.7 / 83.8 and 33.0 / 74.2, so streaming.
+bool bgemm_shared(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn) {
+  if (kn.bgemm_nc) return kn.bgemm_nc == 1;
+  if (batch <= 16) return true;
+  int maxt = 0;
+  for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
+  const bool longk = maxt >= 512;
+  if (f16) return batch <= 64 || (batch <= 512 && !longk);
+  return batch <= 64 && longk && W[0]->codebook != TRELLIS_CB_1MAD;
 }
 
 // Column-block width in 16-column units: 1 up to 16 rows, 2 up to 32; above, the width that
@@ -269,7 +293,7 @@ int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16, const
   long long best_cost = 0;
   for (int nc = batch <= 64 ? 2 : 4; nc <= (batch <= 64 ? 4 : 16); nc *= 2) {
     long long c;
-    bgemm_kr_cost(W, count, batch, nc, f16, true, kn, &c);
+    bgemm_kr_cost(W, count, batch, nc, f16, false, true, kn, &c);
     if (best == 0 || c < best_cost) {
       best = nc;
       best_cost = c;
@@ -302,10 +326,10 @@ bool use_gemv(const trellis_desc* const* W, int count, int batch, const Knobs& k
 // chunks of 32 rows of single values, which take no more than the rows of pairs from 16 rows on
 // (a plan's workspace must not grow past the no-allocation entry point's scratch; fewer rows
 // come here only where the column-block width is forced).
-size_t xf_bytes(int nc, int batch, int k) {
+size_t xf_bytes(bool frag, int batch, int k) {
   const size_t pairs = static_cast<size_t>(batch) * k * 4;
   const size_t frags = static_cast<size_t>((batch + XF_CHUNK - 1) / XF_CHUNK) * (k / 16) * XF_FRAG;
-  return nc > 1 && frags > pairs ? frags : pairs;
+  return frag && frags > pairs ? frags : pairs;
 }
 
 // `split` off: the batched path's k-ranges are whole (no partial sums in the workspace).
@@ -314,9 +338,11 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
   GroupPlan p;
   p.gemv = use_gemv(W, count, batch, kn);
   p.nb = batch;
-  p.nc = bgemm_nc(W, count, batch, f16, kn);
+  p.shared = bgemm_shared(W, count, batch, f16, kn);
+  p.nc = !p.shared ? bgemm_nc(W, count, batch, f16, kn)
+                   : kn.bgemm_nc == 1 || batch <= 16 ? 1 : batch <= 32 ? 2 : batch <= 64 ? 4 : 8;
   p.ncb = p.gemv ? 1 : (batch + 16 * p.nc - 1) / (16 * p.nc);
-  p.kr = p.gemv ? gemv_kr(W, count, batch, kn) : bgemm_kr(W, count, batch, p.nc, f16, split_k, kn);
+  p.kr = p.gemv ? gemv_kr(W, count, batch, kn) : bgemm_kr(W, count, batch, p.nc, f16, p.shared, split_k, kn);
   // tiles per decode-GEMV stage: 16, or 8 for short k-ranges and for launches that split k
   // (a workgroup's first stage lands sooner: the 8B block's q/k/v and down launches
   // 0.2-0.7 us faster each at batch 1 to 8)
@@ -355,7 +381,7 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
       p.ws += align256(static_cast<size_t>(p.n_ob[i]) * p.ncb * p.S[i] * part_cols * 128 *
                        sizeof(float));
     p.off_xf[i] = p.ws;
-    if (!p.gemv) p.ws += align256(xf_bytes(p.nc, p.nb, W[i]->k_in));
+    if (!p.gemv) p.ws += align256(xf_bytes(!p.shared, p.nb, W[i]->k_in));
   }
   return p;
 }
@@ -372,17 +398,22 @@ int launch_gemv(int K, int cb, int V, int kc, const LinArgs& g, hipStream_t st) 
 
 // The x fold of every member (the batched path), written once to the workspace: in rows for
 // 16 batch columns, in MFMA fragments above.
-int launch_xfold(LinArgs& g, int nc, int folds, hipStream_t st) {
+int launch_xfold(LinArgs& g, bool shared, int folds, hipStream_t st) {
   const int items = g.total;
   g.total = folds;
   const bool one = g.nmat == 1;
-  if (nc == 1) {
+  if (shared) {
     const dim3 grid(static_cast<unsigned>((folds + 3) / 4));
-    if (one) hipLaunchKernelGGL((xfold_kernel<true>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((xfold_kernel<false>), grid, dim3(256), 0, st, g);
+    if (xfold_rows(false, g.batch) == 4) {
+      if (one) hipLaunchKernelGGL((xfold_kernel<4, true>), grid, dim3(256), 0, st, g);
+      else hipLaunchKernelGGL((xfold_kernel<4, false>), grid, dim3(256), 0, st, g);
+    } else {
+      if (one) hipLaunchKernelGGL((xfold_kernel<1, true>), grid, dim3(256), 0, st, g);
+      else hipLaunchKernelGGL((xfold_kernel<1, false>), grid, dim3(256), 0, st, g);
+    }
   } else {
     const dim3 grid(static_cast<unsigned>(folds));
-    if (xfold_rows(nc, g.batch) == 32) {
+    if (xfold_rows(true, g.batch) == 32) {
       if (one) hipLaunchKernelGGL((xfold_frag_kernel<4, true>), grid, dim3(512), 0, st, g);
       else hipLaunchKernelGGL((xfold_frag_kernel<4, false>), grid, dim3(512), 0, st, g);
     } else {
@@ -395,13 +426,13 @@ int launch_xfold(LinArgs& g, int nc, int folds, hipStream_t st) {
 }
 
 // The batched path: the x fold, the decode-once batched kernel, and (split-K) its reduction.
-int launch_bgemm(int K, int cb, int V, int nc, LinArgs& g, int folds, int nfold, hipStream_t st) {
-  int v = launch_xfold(g, nc, folds, st);
+int launch_bgemm(int K, int cb, int V, int nc, bool shared, LinArgs& g, int folds, int nfold, hipStream_t st) {
+  int v = launch_xfold(g, shared, folds, st);
   if (v) return v;
   switch (K) {
-    case 2: v = launch_bgemm_k<2>(cb, V, nc, g, st); break;
-    case 3: v = launch_bgemm_k<3>(cb, V, nc, g, st); break;
-    default: v = launch_bgemm_k<4>(cb, V, nc, g, st); break;
+    case 2: v = launch_bgemm_k<2>(cb, V, nc, shared, g, st); break;
+    case 3: v = launch_bgemm_k<3>(cb, V, nc, shared, g, st); break;
+    default: v = launch_bgemm_k<4>(cb, V, nc, shared, g, st); break;
   }
   if (v || nfold == 0) return v;
   return launch_bfold(cb, nc, nfold, g, st);
@@ -770,10 +801,10 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
       g.m[i].x = static_cast<const char*>(x[i]) + static_cast<size_t>(b0) * ldx[i] * xes;
       g.m[i].y = static_cast<char*>(y[i]) + static_cast<size_t>(b0) * ldy[i] * yes;
       g.m[i].chunk0 = chunk0;
-      chunk0 += ((g.batch + xfold_rows(p.nc, g.batch) - 1) / xfold_rows(p.nc, g.batch)) * ((W[i]->k_in + 127) / 128);
+      chunk0 += ((g.batch + xfold_rows(!p.shared, g.batch) - 1) / xfold_rows(!p.shared, g.batch)) * ((W[i]->k_in + 127) / 128);
     }
     v = p.gemv ? launch_gemv(W[0]->K, W[0]->codebook, W[0]->V, p.kc, g, st)
-               : launch_bgemm(W[0]->K, W[0]->codebook, W[0]->V, p.nc, g, chunk0, nfold, st);
+               : launch_bgemm(W[0]->K, W[0]->codebook, W[0]->V, p.nc, p.shared, g, chunk0, nfold, st);
     if (v) return v;
   }
   return TRELLIS_OK;
