@@ -110,7 +110,7 @@ int trellis_workspace_bytes(const trellis_desc *W, int batch, size_t *bytes);
  * Batch 1 to 4 runs one decode-GEMV launch (gemv_kernel, x fold fused; the batch rows
  * ride the MFMA's columns), and so does batch 5 to 16 when that launch's work items fit one
  * round on the CUs. Other calls run the x fold once, then a decode-once batched kernel
- * (bgemm16_kernel, bgemm_kernel or bgemm_wide_kernel: each weight tile decoded once per 16 to
+ * (bgemm_shared_kernel, bgemm_kernel or bgemm_wide_kernel: each weight tile decoded once per 16 to
  * 256 batch columns, as the launch plan chooses, and fed to exact fp16 MFMAs), and, when the
  * launch plan splits k, the slice
  * reduction and output fold (bfold_kernel). */
