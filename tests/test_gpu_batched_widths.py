@@ -48,7 +48,8 @@ def test_widths_at_tile_edges(te, gpu_device, monkeypatch, nc, n, k, K, cb, V, b
 @pytest.mark.parametrize("n,k,K,cb,V,batch,f16", [
     (144, 48, 3, "mcg", 1, 17, True), (272, 336, 2, "3inst", 2, 33, True), (128, 2064, 4, "1mad", 1, 65, True),
     (400, 1040, 3, "mcg", 1, 129, True), (96, 8192, 3, "mcg", 1, 64, True), (144, 528, 4, "mcg", 2, 257, True),
-    (272, 8192, 3, "mcg", 1, 17, False), (128, 8208, 2, "3inst", 2, 64, False)])
+    (272, 8192, 3, "mcg", 1, 17, False), (128, 8208, 2, "3inst", 2, 64, False),
+    (272, 528, 3, "mcg", 1, 65, False), (144, 1024, 2, "3inst", 1, 128, False), (96, 512, 4, "mcg", 1, 700, True)])
 def test_shared_activation_kernel(te, gpu_device, n, k, K, cb, V, batch, f16):
     """The 16-wave kernel above 16 rows, as the planner picks it (fp16-weight mode, and the
     exact mode with a k of 8192 and more), split k and odd tiles included."""

@@ -269,14 +269,18 @@ int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f1
 //   fp16-weight mode, up to 64 rows: block at 32 / 64 rows shared 77.9 / 97.5, streaming 83.5 /
 //   103.1. At 128 / 512 rows, k of 4096: gate+up 47.0 / 154.7 and 54.6 / 162.5, q/k/v 26.7 /
 //   52.2 and 27.8 / 58.6; long k: down 32.7 / 83.8 and 33.0 / 74.2, so streaming.
+//   k up to 1024 (little work per item to pay the streaming kernels' output fold with):
+//   4096x512 + 12160x512 at 100 rows exact shared 15.0 us, streaming 18.8, at 512 exact 50.3 and
+//   45.8; fp16-weight mode at 1982 rows 117 and 134 (2 x 4096x1024: 84 and 92).
 bool bgemm_shared(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn) {
   if (kn.bgemm_nc) return kn.bgemm_nc == 1;
   if (batch <= 16) return true;
   int maxt = 0;
   for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
   const bool longk = maxt >= 512;
-  if (f16) return batch <= 64 || (batch <= 512 && !longk);
-  return batch <= 64 && longk && W[0]->codebook != TRELLIS_CB_1MAD;
+  const bool shortk = maxt <= 64;
+  if (f16) return batch <= 64 || shortk || (batch <= 512 && !longk);
+  return W[0]->codebook != TRELLIS_CB_1MAD && (batch <= 64 ? longk : batch <= 128 && shortk);
 }
 
 // Column-block width in 16-column units: 1 up to 16 rows, 2 up to 32; above, the width that
@@ -340,7 +344,7 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
   p.nb = batch;
   p.shared = bgemm_shared(W, count, batch, f16, kn);
   p.nc = !p.shared ? bgemm_nc(W, count, batch, f16, kn)
-                   : kn.bgemm_nc == 1 || batch <= 16 ? 1 : batch <= 32 ? 2 : batch <= 64 ? 4 : 8;
+                   : kn.bgemm_nc == 1 || batch <= 16 ? 1 : batch <= 32 ? 2 : batch <= 64 || !f16 ? 4 : 8;
   p.ncb = p.gemv ? 1 : (batch + 16 * p.nc - 1) / (16 * p.nc);
   p.kr = p.gemv ? gemv_kr(W, count, batch, kn) : bgemm_kr(W, count, batch, p.nc, f16, p.shared, split_k, kn);
   // tiles per decode-GEMV stage: 16, or 8 for short k-ranges and for launches that split k
