@@ -555,17 +555,21 @@ __device__ __forceinline__ half8_t decode_a(uint32_t wlo, uint32_t whi, int sh) 
   return __builtin_bit_cast(half8_t, a4);
 }
 
-// hi + lo of two codebook pairs (hi in the upper half of each word) as one packed pair of
-// fp16 sums: v_add_f16 with SDWA operand selects, one instruction per value. The fp16 add
-// rounds the exact sum of the two halves to nearest even, as a cast of the reference's
-// fp32 sum (qtip.py:28-29, 45, 53) to fp16 does.
-__device__ __forceinline__ uint32_t add_halves2(uint32_t r0, uint32_t r1) {
-  uint32_t d;
-  asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0\n\t"
-      "v_add_f16_sdwa %0, %2, %2 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1 src1_sel:WORD_0"
-      : "=&v"(d)
-      : "v"(r0), "v"(r1));
-  return d;
+// hi + lo of four codebook pairs (hi in the upper half of each word) as two packed pairs of
+// fp16 sums, r0's and r1's in d0, r2's and r3's in d1: v_add_f16 with SDWA operand selects,
+// one instruction per value. The fp16 add rounds the exact sum of the two halves to nearest
+// even, as a cast of the reference's fp32 sum (qtip.py:28-29, 45, 53) to fp16 does. The two
+// words alternate: gfx940 and later need a wait state between an instruction that writes a
+// part of a register and the next one that reads it (as keeping its other half does), which
+// the compiler's hazard pass does not put inside inline assembly.
+__device__ __forceinline__ void add_halves4(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t r3,
+                                            uint32_t& d0, uint32_t& d1) {
+  asm("v_add_f16_sdwa %0, %2, %2 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0\n\t"
+      "v_add_f16_sdwa %1, %4, %4 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0\n\t"
+      "v_add_f16_sdwa %0, %3, %3 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1 src1_sel:WORD_0\n\t"
+      "v_add_f16_sdwa %1, %5, %5 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1 src1_sel:WORD_0"
+      : "=&v"(d0), "=&v"(d1)
+      : "v"(r0), "v"(r1), "v"(r2), "v"(r3));
 }
 
 // The A operand of a tile pair in the fp16-weight mode (one MAC per weight): k-slots
@@ -588,10 +592,8 @@ __device__ __forceinline__ half8_t decode_a_pair(uint32_t wlo0, uint32_t whi0, u
 #pragma unroll
     for (int w = 0; w < 4; ++w) o[w] = h[2 * w] | (h[2 * w + 1] << 16);
   } else {
-    o[0] = add_halves2(a0[0], a0[1]);
-    o[1] = add_halves2(a0[2], a0[3]);
-    o[2] = add_halves2(a1[0], a1[1]);
-    o[3] = add_halves2(a1[2], a1[3]);
+    add_halves4(a0[0], a0[1], a0[2], a0[3], o[0], o[1]);
+    add_halves4(a1[0], a1[1], a1[2], a1[3], o[2], o[3]);
   }
   return __builtin_bit_cast(half8_t, o);
 }
@@ -606,16 +608,17 @@ __device__ __forceinline__ half8_t decode_a_pair(uint32_t wlo0, uint32_t whi0, u
 template <int CB>
 __device__ __forceinline__ half8_t operand_sum(const uint32_t (&p0)[4], const uint32_t (&p1)[4]) {
   uint32_t o[4];
+  if constexpr (CB == CB_1MAD) {
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const uint32_t a = w < 2 ? p0[2 * w] : p1[2 * w - 4], b = w < 2 ? p0[2 * w + 1] : p1[2 * w - 3];
-    if constexpr (CB == CB_1MAD) {
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t a = w < 2 ? p0[2 * w] : p1[2 * w - 4], b = w < 2 ? p0[2 * w + 1] : p1[2 * w - 3];
       const uint32_t y = __builtin_amdgcn_sad_hi_u8(b, 0u, __builtin_amdgcn_sad_u8(a, 0u, 0x64006400u));
       const half2_t off = {static_cast<_Float16>(-1534.0f), static_cast<_Float16>(-1534.0f)};
       o[w] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, y) + off);
-    } else {
-      o[w] = add_halves2(lop3_pair(a), lop3_pair(b));
     }
+  } else {
+    add_halves4(lop3_pair(p0[0]), lop3_pair(p0[1]), lop3_pair(p0[2]), lop3_pair(p0[3]), o[0], o[1]);
+    add_halves4(lop3_pair(p1[0]), lop3_pair(p1[1]), lop3_pair(p1[2]), lop3_pair(p1[3]), o[2], o[3]);
   }
   return __builtin_bit_cast(half8_t, o);
 }
