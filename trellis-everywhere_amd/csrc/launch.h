@@ -50,10 +50,11 @@ static int launch_bfold_cb(int nc, int nfold, const LinArgs& g, hipStream_t st) 
       if (one) hipLaunchKernelGGL((bfold_kernel<CB, 8, true>), grid, dim3(256), 0, st, g);
       else hipLaunchKernelGGL((bfold_kernel<CB, 8, false>), grid, dim3(256), 0, st, g);
       break;
-    default:
+    case 16:
       if (one) hipLaunchKernelGGL((bfold_kernel<CB, 16, true>), grid, dim3(256), 0, st, g);
       else hipLaunchKernelGGL((bfold_kernel<CB, 16, false>), grid, dim3(256), 0, st, g);
       break;
+    default: return 13;
   }
   return hipGetLastError() == hipSuccess ? 0 : 13;
 }
@@ -123,9 +124,10 @@ static int launch_bgemm_nc(int nc, bool shared, const LinArgs& g, hipStream_t st
       case 1: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 1, F16) break;
       case 2: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 2, F16) break;
       case 4: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 4, F16) break;
-      default:
-        if constexpr (F16) { TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 8, F16) }
-        else return 13;
+      case 8:
+        if constexpr (F16) { TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 8, F16) break; }
+        [[fallthrough]];
+      default: return 13;
     }
     return hipGetLastError() == hipSuccess ? 0 : 13;
   }
@@ -133,7 +135,8 @@ static int launch_bgemm_nc(int nc, bool shared, const LinArgs& g, hipStream_t st
     case 2: TRELLIS_BG_LAUNCH(bgemm_kernel, 512, 2, F) break;
     case 4: TRELLIS_BG_LAUNCH(bgemm_kernel, 512, 4, F) break;
     case 8: TRELLIS_BG_LAUNCH(bgemm_wide_kernel, 256, 8, F) break;
-    default: TRELLIS_BG_LAUNCH(bgemm_wide_kernel, 256, 16, F) break;
+    case 16: TRELLIS_BG_LAUNCH(bgemm_wide_kernel, 256, 16, F) break;
+    default: return 13;
   }
 #undef TRELLIS_BG_LAUNCH
   return hipGetLastError() == hipSuccess ? 0 : 13;

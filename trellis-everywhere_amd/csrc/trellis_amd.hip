@@ -107,6 +107,9 @@ Knobs read_knobs() {
     take("SMALL_BATCH_GEMV", k.small_batch_gemv);
     take("PLAN_LOG", k.plan_log);
   }
+  // a width that no kernel has counts as unset
+  const int nc = k.bgemm_nc;
+  if (nc != 1 && nc != 2 && nc != 4 && nc != 8 && nc != 16) k.bgemm_nc = 0;
   return k;
 }
 
@@ -289,8 +292,7 @@ bool bgemm_shared(const trellis_desc* const* W, int count, int batch, bool f16, 
 // 53.7 and 40.8), else of 64, 128 and 256 (gate+up at 512 rows 246, 205 and 222 us, at 1024
 // rows 472, 395 and 365; o at 256 rows 33.0, 33.5 and 39.5).
 int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn) {
-  const int forced = kn.bgemm_nc;
-  if (forced == 1 || forced == 2 || forced == 4 || forced == 8 || forced == 16) return forced;
+  if (kn.bgemm_nc) return kn.bgemm_nc;
   if (batch <= 16) return 1;
   if (batch <= 32) return 2;
   int best = 0;
