@@ -95,7 +95,8 @@ typedef struct trellis_desc {
   int32_t nwords;            /* 256*K/32 words per tile */
 } trellis_desc;
 
-/* Number of workspace bytes trellis_packed_linear needs for this layer and batch.
+/* Number of workspace bytes that every trellis_packed_linear call of up to `batch` rows of
+ * this layer fits in (a smaller batch can need more than a larger one: this is the most).
  * The workspace must be zero-filled once when allocated; every call leaves its
  * counters at zero again. It belongs to one layer (or one group): its counters sit in a
  * header laid out by the members' shapes alone, so calls at any batch size may share it

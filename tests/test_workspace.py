@@ -1,8 +1,10 @@
 """Host-side workspace sizing of the packed linear (no GPU): a run of growing batch sizes
 replaces the workspace O(log n) times, and the buffers kept alive for captured graphs stay
-smaller together than the current one."""
+smaller together than the current one. The size of a batch covers every smaller one."""
+import ctypes
 import importlib
 
+import pytest
 import torch
 
 from conftest import PKG
@@ -31,3 +33,25 @@ def test_workspace_growth_is_geometric():
     cur = owner._ws
     assert pl._grow_workspace(owner, 100) is cur
     assert pl._ws_size(1) == 256 and pl._ws_size(256) == 256 and pl._ws_size(257) == 512
+
+
+@pytest.mark.parametrize("knob", [None, ("TRELLIS_BGEMM_NC", "1"), ("TRELLIS_BGEMM_NC", "2"),
+                                  ("TRELLIS_BGEMM_NC", "16"), ("TRELLIS_SMALL_BATCH_GEMV", "0")])
+@pytest.mark.parametrize("shapes", [((4096, 4096),), ((7584, 848),), ((4096, 12288),), ((512, 512),), ((16, 16),),
+                                    ((4096, 4096), (1024, 4096), (1024, 4096)), ((272, 336), (1040, 2064))])
+def test_size_covers_every_smaller_batch(te, monkeypatch, shapes, knob):
+    """Calls check their own plan's need, which a query at that batch never reports less than:
+    sizes that never fall with the batch cover every smaller call."""
+    lib = te.library()
+    if knob:
+        monkeypatch.setenv(*knob)
+    for codebook in (0, 2):
+        descs = [te._capi.TrellisDesc(bits=16, su=16, sv=16, isc_scaled=16, osc=16, n_out=n, k_in=k, K=3, V=1,
+                                      codebook=codebook, block_in=16, block_out=16, nwords=24)
+                 for n, k in shapes]
+        ptrs = (ctypes.POINTER(te._capi.TrellisDesc) * len(descs))(*[ctypes.pointer(d) for d in descs])
+        need, last = ctypes.c_size_t(0), 0
+        for batch in (*range(1, 300), 383, 384, 385, 511, 512, 513, 576, 577, 1023, 1024, 1025, 2048, 2049, 5000):
+            te._capi.check(lib.trellis_workspace_bytes_group(ptrs, len(descs), batch, ctypes.byref(need)))
+            assert need.value >= last, (batch, need.value, last)
+            last = need.value

@@ -392,6 +392,26 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
   return p;
 }
 
+// Workspace bytes that cover every call of up to `batch` rows, in either MFMA mode (their
+// k-ranges, hence partial buffers, may differ). A smaller batch can need more: fewer column
+// blocks leave CUs idle that a split of k then fills (4096 x 4096 at K=3: 25.2 MB at 512 rows,
+// 8.4 MB at 513). A plan's choices change with the batch only at 1, 2, 4, 8, 16, 32 and 64 rows
+// and where another column block starts, 64 columns or more apart above 64 rows; up to the next
+// such end it grows with the rows, so only the ends and `batch` itself are planned.
+size_t covering_ws(const trellis_desc* const* W, int count, int batch, const Knobs& kn) {
+  const int step = kn.bgemm_nc == 1 ? 16 : kn.bgemm_nc == 2 ? 32 : 64;
+  size_t most = 0;
+  for (int b = 1;;) {
+    const int at = b < batch ? b : batch;
+    for (const bool f16 : {false, true}) {
+      const size_t ws = group_plan(W, count, at, f16, kn).ws;
+      most = ws > most ? ws : most;
+    }
+    if (at == batch) return most;
+    b = b < step ? 2 * b : b > batch - step ? batch : b + step;
+  }
+}
+
 // The pipelined decode-GEMV (its x fold is fused): batch 1 to 4, and 5 to 16 where
 // use_gemv picks it.
 int launch_gemv(int K, int cb, int V, int kc, const LinArgs& g, hipStream_t st) {
@@ -557,10 +577,7 @@ int trellis_workspace_bytes_group(const trellis_desc* const* W, int count, int b
   const int v = validate_group(W, count);
   if (v) return v;
   if (batch < 1) return TRELLIS_ERR_BATCH;
-  // either MFMA mode's plan fits (their k-ranges, hence partial buffers, may differ)
-  const Knobs kn = read_knobs();
-  const size_t a = group_plan(W, count, batch, false, kn).ws, b = group_plan(W, count, batch, true, kn).ws;
-  *bytes = a > b ? a : b;
+  *bytes = covering_ws(W, count, batch, read_knobs());
   return TRELLIS_OK;
 }
 
