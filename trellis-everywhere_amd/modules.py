@@ -53,11 +53,14 @@ class TrellisLinear(torch.nn.Module):
             y = self.packed.forward(x2, out_dtype=out_dtype, mma_f16=self.mma_f16)
         bias = self.bias
         if bias is not None:
+            done = None
             if x.dtype == torch.bfloat16 and not bias.requires_grad:
                 # the fp32 sum rounded once as it is stored: one kernel, not an add and a cast
-                y = torch.add(y, bias, out=torch.empty(y.shape, dtype=x.dtype, device=y.device))
-            else:
-                y = y + bias.to(y.dtype)
+                try:
+                    done = torch.add(y, bias, out=torch.empty(y.shape, dtype=x.dtype, device=y.device))
+                except RuntimeError:
+                    pass   # vmap and forward-mode differentiation over the bias take no out=
+            y = y + bias.to(y.dtype) if done is None else done
         return y.to(x.dtype).reshape(*lead, self.out_features)
 
     def extra_repr(self) -> str:
