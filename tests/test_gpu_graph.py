@@ -31,8 +31,7 @@ def make_linear(te, bits, rec, device):
                                               (64, False, None), (64, True, None),
                                               (200, False, None), (200, False, "8")])
 def test_graph_replays_match_eager(te, gpu_device, monkeypatch, batch, mma_f16, nc):
-    """nc forces the batched kernel's column-block width (8 chunks: the exact mode's
-    two-wave 128-column kernel)."""
+    """nc forces the column-block width (8: bgemm_wide_kernel's blocks of 128 columns)."""
     _say(f"[graph] batch={batch} mma_f16={mma_f16} nc={nc}")
     if nc is not None:
         monkeypatch.setenv("TRELLIS_BGEMM_NC", nc)

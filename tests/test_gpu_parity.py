@@ -290,11 +290,10 @@ def test_prefill_ragged_fold_rows(te, gpu_device, batch):
 @pytest.mark.parametrize("K,cb,V", [(2, "mcg", 1), (3, "mcg", 1), (4, "mcg", 1), (3, "3inst", 2),
                                     (3, "1mad", 1), (4, "3inst", 1), (2, "1mad", 2)])
 def test_prefill_column_block_width(te, gpu_device, monkeypatch, K, cb, V):
-    """Above 64 columns the batched kernel runs 64-column blocks (16 waves) or, as the
-    planner's cost model decides, 128-column blocks (8 waves in the exact mode, whose
-    fragments and accumulators need two waves' worth of registers). Every width, forced
-    with TRELLIS_BGEMM_NC in either mode, gives the oracle's result, and the exact mode's
-    widths agree to fp32 summation order."""
+    """Above 64 rows the planner chooses the kernel and its column-block width. Blocks of 64
+    columns (bgemm_kernel) and of 128 (bgemm_wide_kernel), forced with TRELLIS_BGEMM_NC in
+    either mode, give the oracle's result, and the exact mode's widths agree with the planned
+    launch to fp32 summation order."""
     _say(f"[prefill width] K={K} cb={cb} V={V} batch=200")
     bits, rec = tn.synthetic_record(512, 1024, K, seed=200 + K, codebook=cb, V=V)
     lin = make_linear(te, bits, rec, gpu_device)
