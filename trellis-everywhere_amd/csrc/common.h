@@ -47,14 +47,15 @@ struct alignas(64) LinMat {
   int n, block_in, k, block_out;
   float nrm_in, nrm_out;  // 1 / sqrt(block_in), 1 / sqrt(block_out), rounded as fp32 ops
   int n_ob;
-  int xfw;              // words per xf row: k ((x, x) fp16 pairs), or kp / 2 in the fp16-weight
-                        // mode (kp = k rounded up to 32; fp16 values, tile pairs interleaved)
+  int xfw;              // words per xf row in the row layout: k ((x, x) fp16 pairs), or kp / 2 in the
+                        // fp16-weight mode (kp = k rounded up to 32; fp16 values, tile pairs interleaved)
   long long ldx, ldy;
   void* y;
   float* part;          // workspace: split-K partial sums (S > 1)
   // ---- third line
   unsigned* tickets;    // workspace: [n_ob] arrival counters (batch 1, S > 1), zero between calls
-  uint32_t* xf;         // workspace: [batch][xfw words] folded activations (xfold_kernel)
+  uint32_t* xf;         // workspace: folded activations, [batch][xfw words] (xfold_kernel) or 32-row
+                        // chunks of MFMA fragments (xfold_frag_kernel)
   int chunk0;           // first group-wide x-fold job of this matrix
   int fold0;            // first group-wide bfold_kernel job of this matrix
   int y_words;          // every row of y starts at a 4-byte aligned address
@@ -391,7 +392,7 @@ __device__ __forceinline__ int xf_pair_slot(int e) {
 // ---------------------------------------------------------------- x fold
 // xf = Hb_k(isc * su * x) scaled by 1/sqrt(block_in), once per batched call.
 //
-// Above 16 rows, the kernels' B layout: chunks of 32 batch rows, each
+// For the streaming kernels, their B layout: chunks of 32 batch rows, each
 // [tile column][h = 0, 1][32 rows] of 16 bytes holding the fp16 values of columns 4h .. 4h+3
 // and 8+4h .. 8+4h+3 of the tile: the 1 KB of a (chunk, tile column) is one fragment of
 // v_mfma_f32_32x32x16_f16, lane l = (row l % 32, h = l / 32), read as one coalesced load.
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(512) void xfold_frag_kernel(LinArgs g) {
   }
 }
 
-// The x fold for the 16-row kernel: rows of (x, x) fp16 pairs, or in the fp16-weight mode of
+// The x fold for bgemm_shared_kernel: rows of (x, x) fp16 pairs, or in the fp16-weight mode of
 // fp16 values in tile-pair order (xf_pair_slot). One wave per (matrix, batch row, 128-column
 // chunk), every load a range-checked buffer load issued up front: a few rows are latency-
 // bound, and one row per wave gives every SIMD several waves to overlap the transform's
