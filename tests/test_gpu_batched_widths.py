@@ -50,10 +50,11 @@ def test_widths_at_tile_edges(te, gpu_device, monkeypatch, nc, n, k, K, cb, V, b
     (400, 1040, 3, "mcg", 1, 129, True), (96, 8192, 3, "mcg", 1, 64, True), (144, 528, 4, "mcg", 2, 257, True),
     (272, 8192, 3, "mcg", 1, 17, False), (128, 8208, 2, "3inst", 2, 64, False),
     (272, 528, 3, "mcg", 1, 65, False), (144, 1024, 2, "3inst", 1, 128, False), (96, 512, 4, "mcg", 1, 700, True)])
-def test_shared_activation_kernel(te, gpu_device, n, k, K, cb, V, batch, f16):
-    """The 16-wave kernel above 16 rows, as the planner picks it (fp16-weight mode, and the
-    exact mode with a k of 8192 and more), split k and odd tiles included."""
+def test_shared_activation_kernel(te, gpu_device, monkeypatch, capfd, n, k, K, cb, V, batch, f16):
+    """bgemm_shared_kernel above 16 rows, where the planner picks it (as its log says), split k
+    and odd tiles included."""
     print(f"[shared] n={n} k={k} K={K} cb={cb} V={V} batch={batch} f16={f16}", flush=True)
+    monkeypatch.setenv("TRELLIS_PLAN_LOG", "1")
     bits, rec = tn.synthetic_record(n, k, K, seed=n + k, codebook=cb, V=V)
     lin = te.PackedLinear(te.PackedRecord(rec.n, rec.k, rec.K, bits, rec.su, rec.sv, rec.isc, rec.osc,
                                           float(rec.scale), codebook=rec.codebook, V=rec.V),
@@ -61,5 +62,29 @@ def test_shared_activation_kernel(te, gpu_device, n, k, K, cb, V, batch, f16):
     x = np.random.default_rng(batch).standard_normal((batch, k)).astype(np.float16)
     xt = torch.from_numpy(x).to(gpu_device)
     y = lin(xt, mma_f16=f16)
+    assert "shared=1" in capfd.readouterr().err
     assert tn.rel_err(y.cpu().numpy(), tn.packed_linear_ref(bits, rec, x)) < TOL
     assert torch.equal(y, lin(xt, mma_f16=f16))
+
+
+@pytest.mark.parametrize("kr", ["0", "24"])      # the planner's, and one that splits the longer k
+@pytest.mark.parametrize("n,k,K,cb,V,batch", [(12304, 336, 3, "mcg", 1, 129), (4112, 528, 2, "3inst", 2, 760)])
+def test_shared_exact_128_columns(te, gpu_device, monkeypatch, capfd, kr, n, k, K, cb, V, batch):
+    """Its 12-wave instantiation (exact mode, 128 columns, steps of 6 tile columns), single and in
+    a group, with k-ranges that end inside a step and ragged last column blocks."""
+    print(f"[shared 128] n={n} k={k} K={K} cb={cb} V={V} batch={batch} kr={kr}", flush=True)
+    monkeypatch.setenv("TRELLIS_PLAN_LOG", "1")
+    monkeypatch.setenv("TRELLIS_BGEMM_KR", kr)
+    bits, rec = tn.synthetic_record(n, k, K, seed=n + k, codebook=cb, V=V)
+    lin = te.PackedLinear(te.PackedRecord(rec.n, rec.k, rec.K, bits, rec.su, rec.sv, rec.isc, rec.osc,
+                                          float(rec.scale), codebook=rec.codebook, V=rec.V),
+                          device=gpu_device)
+    grp = te.PackedGroup([lin, lin])
+    x = np.random.default_rng(batch).standard_normal((batch, k)).astype(np.float16)
+    xt = torch.from_numpy(x).to(gpu_device)
+    y = lin(xt)
+    log = capfd.readouterr().err
+    assert "shared=1" in log and " nc=8 " in log, log
+    assert tn.rel_err(y.cpu().numpy(), tn.packed_linear_ref(bits, rec, x)) < TOL
+    ys = grp([xt, xt])
+    assert torch.equal(ys[0], ys[1]) and tn.rel_err(ys[0].cpu().numpy(), y.cpu().numpy()) < 1e-5

@@ -55,3 +55,28 @@ def test_size_covers_every_smaller_batch(te, monkeypatch, shapes, knob):
             te._capi.check(lib.trellis_workspace_bytes_group(ptrs, len(descs), batch, ctypes.byref(need)))
             assert need.value >= last, (batch, need.value, last)
             last = need.value
+
+
+@pytest.mark.parametrize("shapes", [((4096, 4096),), ((12304, 336),), ((4864, 896), (4864, 896)), ((2048, 8192),),
+                                    ((272, 336), (1040, 2064))])
+def test_calls_fit_the_size(te, monkeypatch, shapes):
+    """Every smaller call, in either mode and output type (which choose the kernel), passes the
+    library's size check with the size of 700 rows; the address it is given is refused next
+    (TRELLIS_ERR_ALIGN, 8), before anything is launched."""
+    lib, n = te.library(), len(shapes)
+    for codebook in (0, 2):
+        descs = [te._capi.TrellisDesc(bits=16, su=16, sv=16, isc_scaled=16, osc=16, n_out=no, k_in=k, K=3, V=1,
+                                      codebook=codebook, block_in=16, block_out=16, nwords=24)
+                 for no, k in shapes]
+        ptrs = (ctypes.POINTER(te._capi.TrellisDesc) * n)(*[ctypes.pointer(d) for d in descs])
+        at = (ctypes.c_void_p * n)(*[16] * n)
+        ldx = (ctypes.c_int64 * n)(*[k for _, k in shapes])
+        ldy = (ctypes.c_int64 * n)(*[no for no, _ in shapes])
+        need = ctypes.c_size_t(0)
+        te._capi.check(lib.trellis_workspace_bytes_group(ptrs, n, 700, ctypes.byref(need)))
+        for batch in range(1, 701):
+            for ydt in (te._capi.DT_F32, te._capi.DT_F16):
+                for flags in (0, te._capi.MMA_F16):
+                    st = lib.trellis_packed_linear_group_ex(ptrs, n, at, ldx, batch, te._capi.DT_F16, at, ldy, ydt,
+                                                            16, need.value, flags, None)
+                    assert st == 8, (batch, ydt, flags, st)

@@ -1,8 +1,9 @@
 // bgemm.h — batched packed linear for gfx950: decode once, reuse across the batch. Three
 // kernels by the call's rows, each a 128-row output block (the out-dim Hadamard block) x a
 // block of batch columns x one k-range per workgroup, one workgroup per CU:
-//   bgemm_shared_kernel 16 waves, activations shared through LDS: up to 16 rows, and above
-//                     where the planner's rule finds it faster (bgemm_shared);
+//   bgemm_shared_kernel 16 to 128 columns: 16 waves (12 for exact 128-column blocks), activations
+//                     shared through LDS: up to 16 rows, and above where the planner's rule
+//                     finds it faster (streams, trellis_amd.hip);
 //   bgemm_kernel      32 or 64 columns: 8 waves, each with its own share of the k-range;
 //   bgemm_wide_kernel 128 or 256 columns: 4 waves with 64 accumulator tiles each.
 // In each a wave decodes a tile once, straight into the A operand of an MFMA (common.h), and
@@ -12,9 +13,8 @@
 // inside the kernel leaves the whole reduction to the last workgroup of each block, behind
 // device-scope round trips, and measured slower.
 //
-// Measured on the Qwen3-8B block (K=3, MCG, one MI355X, the two sides in turn on one box; the
-// one before is a 16-wave workgroup, 12 for exact 128-column blocks, whose waves shared B tiles
-// double-buffered in LDS with a barrier per step of 6 to 8 tile columns):
+// Measured on the Qwen3-8B block (K=3, MCG, one MI355X, weights from the last-level cache where
+// they fit, in turn on one box), bgemm_shared_kernel and the streaming two:
 //   gate+up, 32 / 64 / 128 rows, exact            32.6 / 42-44 / 68.2 -> 28.3 / 38.5 / 64.9 us
 //   gate+up, 512 rows, exact                      229-235 -> 205-208 us
 //   down, 2048 rows, exact / fp16-weight mode     438-445 / 280-289 -> 333-342 / 236-240 us
@@ -103,7 +103,7 @@ __device__ __forceinline__ void setprio_n(int v) {
 }
 
 // ---------------------------------------------------------------- shared activations
-// A workgroup of 16 waves: wave w = (band group bg = w % NG, k-lane kl = w / NG), a band group
+// A workgroup of 16 (or 12) waves: wave w = (band group bg = w % NG, k-lane kl = w / NG), a band group
 // being BW adjacent bands; the waves of a SIMD share a band group and split every k-step's
 // tiles between them (tile j of a step belongs to k-lane j % KL):
 //   * the B tile of a step (xf[batch cols][KT*16] as (x, x) fp16 pairs written by
@@ -119,14 +119,22 @@ __device__ __forceinline__ void setprio_n(int v) {
 //   * the epilogue adds the k-lanes' sums into t[16 NC][128] in LDS in k-lane order.
 // At 16 rows the kernels below measured slower (8B gate+up 28.9 us with 32-column
 // blocks, 26.5 with this one; q/k/v 16.5 and 15.9, o 14.7 and 13.2, down 19.5 and 17.3).
+//
+// Waves per workgroup: 16 (four per SIMD), or 12 (three per SIMD, up to 168 registers each) for
+// the exact mode's 128-column blocks, whose 8 fragments and 16 accumulators per wave (~150
+// registers) do not fit a quarter of a SIMD's registers.
+template <int NC, int F16> struct BgShared {
+  static constexpr int WAVES = !F16 && NC == 8 ? 12 : 16;
+};
+
 template <int K, int CB, int V, int NC, int F16, bool SINGLE>
-__global__ __launch_bounds__(1024) void bgemm_shared_kernel(LinArgs g) {
-  constexpr int BG_WAVES = 16;
-  static_assert(F16 || NC <= 4, "exact mode: up to 64 columns");
+__global__ __launch_bounds__((64 * BgShared<NC, F16>::WAVES)) void bgemm_shared_kernel(LinArgs g) {
+  constexpr int BG_WAVES = BgShared<NC, F16>::WAVES;
   constexpr int NWK = 8 * K;
   // tile columns per k-step: at 16 columns 16 (half the barriers of 8; the 8B gate+up group 29.1 -> 27.9 us),
-  // otherwise 8 (in the fp16-weight mode a pair per k-lane)
-  constexpr int KT = F16 || NC > 1 ? 8 : 16;
+  // otherwise 8 (in the fp16-weight mode a pair per k-lane), or 6 for the exact mode's 128
+  // columns (two per k-lane over three k-lanes; LDS holds two B steps)
+  constexpr int KT = F16 ? 8 : NC == 1 ? 16 : NC <= 4 ? 8 : 6;
   // bands per wave: at 16 columns 4 (8 k-lanes; each B fragment read from LDS feeds 4 bands: 27.8 ->
   // 26.6-27.1 us), otherwise 2
   constexpr int BW = F16 || NC > 1 ? 2 : 4;
@@ -784,7 +792,7 @@ template <int K, int CB, int V, int NC, int F16, bool SINGLE>
 __global__ __launch_bounds__(256) void bgemm_wide_kernel(LinArgs g) {
   using Sh = BgWide<NC>;
   constexpr int BW = Sh::BW, KL = Sh::KL, T = Sh::T, PB = Sh::PB, NS = Sh::NS, WAVES = Sh::WAVES;
-  constexpr int NB = 16 * NC, XQ = NC / 2;      // batch columns, 32-row chunks of B
+  constexpr int XQ = NC / 2;                    // 32-row chunks of B
   constexpr int NWK = 8 * K, CPT = 2 * K;       // words, 16-byte chunks per tile
   constexpr int BCH = BW * T * CPT, BL = (BCH + 63) / 64, BST = BL * 256;
   constexpr int XL = 2 * XQ, XST = XL * 256;    // loads, words of a B slot (one tile pair)

@@ -124,9 +124,7 @@ static int launch_bgemm_nc(int nc, bool shared, const LinArgs& g, hipStream_t st
       case 1: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 1, F16) break;
       case 2: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 2, F16) break;
       case 4: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 4, F16) break;
-      case 8:
-        if constexpr (F16) { TRELLIS_BG_LAUNCH(bgemm_shared_kernel, 1024, 8, F16) break; }
-        [[fallthrough]];
+      case 8: TRELLIS_BG_LAUNCH(bgemm_shared_kernel, (64 * BgShared<8, F16>::WAVES), 8, F16) break;
       default: return 13;
     }
     return hipGetLastError() == hipSuccess ? 0 : 13;

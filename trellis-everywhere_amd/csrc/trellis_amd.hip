@@ -123,7 +123,6 @@ struct GroupPlan {
   int kr;              // gemv / bgemm: tile columns per k-range
   int kc;              // gemv: tile columns per pipeline stage (8 or 16)
   int total;           // work items over the group
-  int folds;           // x-fold jobs over the group
   int n_ob[MAX_GROUP], S[MAX_GROUP];
   size_t off_tickets[MAX_GROUP], off_part[MAX_GROUP], off_xf[MAX_GROUP];
   size_t header;       // bytes of the ticket header at the start of the workspace
@@ -191,48 +190,59 @@ int gemv_kr(const trellis_desc* const* W, int count, int batch, const Knobs& kn)
 
 // The batched kernels (bgemm.h): NC 16-column batch chunks per workgroup, a work item being one
 // 128-row block x one column block x one k-range of kr tile columns, a multiple of the
-// kernel's step (16 tiles for the 16-row kernel in the exact mode, else 8: a tile per wave at
-// 32 and 64 columns, a pair at 128). The model of a launch, in ns: rounds of items over the
-// CUs x (2 kr band-tiles per SIMD x the time of one + what an item costs besides: start-up,
-// the k-lanes' meeting, output fold), plus, with split-K, the bfold_kernel launch and the
-// partial blocks it moves. The constants follow the kernels' stamped loops and a sweep of
-// every width on the 8B block's launches and a 2048 x 2048 layer at 48 to 2048 rows in both
-// modes, where the width chosen is on average 0.8 % slower than the fastest one (at worst
-// 13 %: q/k/v at 512 rows in the fp16-weight mode). TRELLIS_BGEMM_KR forces a k-range,
-// TRELLIS_BGEMM_NC the width.
+// kernel's step (bgemm_shared_kernel in the exact mode: 16 tiles at 16 columns, 6 at 128;
+// else 8: a tile per wave at 32 and 64 columns, a pair at 128). The model of a launch:
+// rounds of items over the CUs x (2 kr band-tiles per SIMD x the time of one + what an
+// item costs besides: start-up, the k-lanes' meeting, output fold), plus, with split-K, the
+// bfold_kernel launch and the partial blocks it moves. The constants follow the kernels' stamped
+// loops and sweeps of every width. TRELLIS_BGEMM_KR forces a k-range, TRELLIS_BGEMM_NC the width.
 struct BgCost {
-  int tile, item;   // ns per band-tile and SIMD, ns per item
+  int tile, item, fold, bytes;   // per band-tile and SIMD, per item, per split-K launch; bytes of
+                                 // partial blocks per unit
 };
-BgCost bgemm_cost(int nc, bool sum) {
+// In ns; bgemm_shared_kernel's above 16 columns in cycles at 2.4 GHz (one kernel's costs are compared
+// with each other only).
+BgCost bgemm_cost(int nc, bool shared, bool f16, bool sum) {
   // sum: one fp16 per weight (the fp16-weight mode, 1MAD); above 64 columns two MACs per
   // weight cost their time, up to 64 the decode and its issue set it
+  if (nc == 1) return {33, 2600, 3500, 4500};
+  if (shared) return {f16 ? 75 + 10 * nc : nc == 8 ? 225 : 61 + 19 * nc, 3600, 3600, 1250};
   switch (nc) {
-    case 1: return {33, 2600};
-    case 2: return sum ? BgCost{38, 3000} : BgCost{40, 3000};
-    case 4: return sum ? BgCost{50, 6000} : BgCost{58, 6100};
-    case 8: return sum ? BgCost{76, 8700} : BgCost{93, 8800};
-    default: return sum ? BgCost{116, 18000} : BgCost{150, 18000};
+    case 2: return {sum ? 38 : 40, 3000, 3500, 4500};
+    case 4: return sum ? BgCost{50, 6000, 3500, 4500} : BgCost{58, 6100, 3500, 4500};
+    case 8: return sum ? BgCost{76, 8700, 3500, 4500} : BgCost{93, 8800, 3500, 4500};
+    default: return {sum ? 116 : 150, 18000, 3500, 4500};
   }
 }
 
-// Largest k-range with `split` off: one per block.
-int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool shared,
-                  bool split, const Knobs& kn, long long* cost) {
+// One of the batched kernels on a call: its column-block width and k-range, and what the
+// launch then comes to.
+struct BgPlan {
+  bool shared = false;
+  int nc = 0, kr = 0, smax = 1;      // most k-ranges of a member
+  long long cost = -1, rounds = 0, part_bytes = 0;
+};
+
+// `split` off: one k-range per block.
+BgPlan bgemm_plan(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool shared,
+                  bool split, const Knobs& kn) {
   int maxt = 0;
   for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
-  const int kt = nc == 1 && !f16 ? 16 : 8;
-  // (bgemm_shared_kernel above 16 rows: its step costs and launch terms, in ns at 2.4 GHz)
-  const bool row = shared && nc > 1;
-  const BgCost bc = row ? BgCost{(f16 ? 75 + 10 * nc : 61 + 19 * nc) * 10 / 24, 1500}
-                        : bgemm_cost(nc, f16 || W[0]->codebook == TRELLIS_CB_1MAD);
+  const int kt = f16 ? 8 : nc == 1 ? 16 : shared && nc == 8 ? 6 : 8;
+  const BgCost bc = bgemm_cost(nc, shared, f16, f16 || W[0]->codebook == TRELLIS_CB_1MAD);
   const int cap = ((maxt + kt - 1) / kt) * kt;
   const long long cus = device_cus();
   const long long ncb = (batch + 16 * nc - 1) / (16 * nc);
   const int forced = kn.bgemm_kr;
   const bool force = split && forced >= kt && forced % kt == 0;
-  int best = cap;
-  long long best_cost = -1;
-  for (int kr = !split ? cap : force ? (forced < cap ? forced : cap) : kt; kr <= cap; kr += kt) {
+  BgPlan best;
+  // members of one k: of the k-ranges that cut it into S slices the shortest is the cheapest, so
+  // those of S = 16 .. 1 are looked at (a call's host time pays for the search)
+  bool one_k = true;
+  for (int i = 1; i < count; ++i) one_k = one_k && W[i]->k_in == W[0]->k_in;
+  const auto shortest = [&](int S) { return ((maxt + S - 1) / S + kt - 1) / kt * kt; };
+  int S1 = 16;
+  for (int kr = !split ? cap : force ? (forced < cap ? forced : cap) : one_k ? shortest(S1) : kt; kr <= cap;) {
     long long items = 0, part_bytes = 0;
     int smax = 1;
     for (int i = 0; i < count; ++i) {
@@ -242,70 +252,132 @@ int bgemm_kr_cost(const trellis_desc* const* W, int count, int batch, int nc, bo
       smax = S > smax ? S : smax;
       if (S > 1) part_bytes += static_cast<long long>(S) * n_ob * ncb * 128 * 16 * nc * 4;
     }
-    if (smax > 16 && !force) continue;
     const long long rounds = (items + cus - 1) / cus;
     const long long c = rounds * (2LL * kr * bc.tile + bc.item) +
-                        (smax > 1 ? (row ? 1500 + part_bytes / 3000 : 3500 + part_bytes / 4500) : 0);
-    if (best_cost < 0 || c < best_cost) {
-      best = kr;
-      best_cost = c;
-    }
-    if (force) break;
+                        (smax > 1 ? bc.fold + part_bytes / bc.bytes : 0);
+    if ((smax <= 16 || force) && (best.cost < 0 || c < best.cost))
+      best = {shared, nc, kr, smax, c, rounds, part_bytes};
+    if (force || kr == cap) break;
+    int next = kr + kt;
+    if (one_k)
+      while (S1 > 1 && (next = shortest(--S1)) == kr) {}
+    kr = next;
   }
-  *cost = best_cost;
   return best;
 }
 
-int bgemm_kr(const trellis_desc* const* W, int count, int batch, int nc, bool f16, bool shared,
-             bool split, const Knobs& kn) {
-  long long cost;
-  return bgemm_kr_cost(W, count, batch, nc, f16, shared, split, kn, &cost);
+// The cheapest of the widths lo, 2 lo, .. hi (in 16-column units) by the model.
+BgPlan bgemm_cheapest(const trellis_desc* const* W, int count, int batch, int lo, int hi, bool f16,
+                      bool shared, bool split, const Knobs& kn) {
+  BgPlan best;
+  for (int nc = lo; nc <= hi; nc *= 2) {
+    const BgPlan p = bgemm_plan(W, count, batch, nc, f16, shared, split, kn);
+    if (best.nc == 0 || p.cost < best.cost) best = p;
+  }
+  return best;
+}
+
+// bgemm_shared_kernel's widths: 16 columns up to 16 rows, 32 up to 32 rows, then the cheaper of
+// 32 and 64 up to 64 rows (4096x512 + 12160x512 at 64 rows 12.3 and 14.4 us, the 8B down 29.4 and
+// 26.6), above the cheaper of 64 and 128 (1MAD in the fp16-weight mode: 128, its decode costs more:
+// gate+up at 300 rows 162 and 176).
+BgPlan plan_shared(const trellis_desc* const* W, int count, int batch, bool f16, bool split, const Knobs& kn) {
+  const int lo = kn.bgemm_nc == 1 || batch <= 16 ? 1 : batch <= 64 ? 2
+                 : f16 && W[0]->codebook == TRELLIS_CB_1MAD ? 8 : 4;
+  const int hi = lo == 1 ? 1 : batch <= 32 ? 2 : batch <= 64 ? 4 : 8;
+  return bgemm_cheapest(W, count, batch, lo, hi, f16, true, split, kn);
+}
+
+// The streaming kernels' (bgemm_kernel, bgemm_wide_kernel): 32 columns up to 32 rows, the cheaper of
+// 32 and 64 up to 64 rows (at 64 rows the 8B o launch takes 17.5 us in 32-column blocks and 19.7
+// in 64-column ones, gate+up 53.7 and 40.8), above of 64, 128 and 256 (gate+up at 512 rows 246,
+// 205 and 222 us, at 1024 rows 472, 395 and 365; o at 256 rows 33.0, 33.5 and 39.5).
+BgPlan plan_streaming(const trellis_desc* const* W, int count, int batch, bool f16, bool split, const Knobs& kn) {
+  const int forced = kn.bgemm_nc;
+  const int lo = forced ? forced : batch <= 64 ? 2 : 4;
+  const int hi = forced ? forced : batch <= 32 ? 2 : batch <= 64 ? 4 : 16;
+  return bgemm_cheapest(W, count, batch, lo, hi, f16, false, split, kn);
+}
+
+// ns of a whole call above 64 rows, x fold included, for the choice between the two: fitted to
+// launches of 32 shapes, k of 512 to 14336, 80 to 1982 rows, K = 2, 3 and 4, each kernel at its
+// planned width (362 in each mode with f32 outputs, 135 with f16; mean error 6 %). The streaming
+// kernels' output fold stores 16 bytes a lane, which f32 rows leave in half as long runs.
+long long call_ns(const BgPlan& p, bool f16, bool y_f16) {
+  struct Time { int tile, item; };
+  static constexpr Time SHARED[2][2] = {{{73, 9700}, {125, 10900}}, {{60, 9700}, {77, 11400}}};   // [mode][64, 128 columns]
+  static constexpr Time STREAM[2][2][3] = {{{{66, 11700}, {95, 18100}, {176, 28100}},             // [y][mode][64, 128, 256]
+                                            {{53, 11900}, {72, 17300}, {120, 28700}}},
+                                           {{{61, 9400}, {99, 12000}, {180, 14300}},
+                                            {{49, 9700}, {73, 12200}, {125, 14800}}}};
+  const Time t = p.shared ? SHARED[f16][p.nc > 4] : STREAM[y_f16][f16][p.nc > 8 ? 2 : p.nc > 4];
+  return p.rounds * (2LL * p.kr * t.tile + t.item) + p.part_bytes / (p.shared ? 3000 : y_f16 ? 1900 : 5000);
 }
 
 // Which batched kernel above 16 rows: bgemm_shared_kernel (16 waves, B shared through LDS), or
-// the streaming ones. With weights that come from HBM (a model's, 14 copies of the 8B block in
-// turn, K=3 MCG) the shared one's four waves per SIMD hide more of the loads' latency, and the
-// streaming ones have cheaper products:
-//   exact, up to 64 rows, long k that is split: down (768 tile columns) at 32 / 64 rows shared
-//   20.2 / 26.6 us, streaming 20.9 / 29.4; shorter k at 64 rows q/k/v 22.3 and 21.8, o 16.9 and
-//   16.7, gate+up 41.3 and 40.9 (34.7 with its weights in the last-level cache).
-//   fp16-weight mode, up to 64 rows: block at 32 / 64 rows shared 77.9 / 97.5, streaming 83.5 /
-//   103.1. At 128 / 512 rows, k of 4096: gate+up 47.0 / 154.7 and 54.6 / 162.5, q/k/v 26.7 /
-//   52.2 and 27.8 / 58.6; long k: down 32.7 / 83.8 and 33.0 / 74.2, so streaming.
-//   k up to 1024 (little work per item to pay the streaming kernels' output fold with):
-//   4096x512 + 12160x512 at 100 rows exact shared 15.0 us, streaming 18.8, at 512 exact 50.3 and
-//   45.8; fp16-weight mode at 1982 rows 117 and 134 (2 x 4096x1024: 84 and 92).
-bool bgemm_shared(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn) {
-  if (kn.bgemm_nc) return kn.bgemm_nc == 1;
-  if (batch <= 16) return true;
+// the streaming ones, whose products are cheaper and whose start-up and output fold cost more.
+// Both measured with weights from HBM (24 copies, or 0.5 GB, in turn), us, shared and streaming:
+//   Up to 64 rows the four waves per SIMD hide more of the loads' latency: down at 40 rows 23.1 and
+//   26.4, 16384x2048 at 32 rows 17.2 and 18.7, 8192x8192 at 64 rows 29.6 and 31.0. Not in the
+//   exact mode where a group's whole k-ranges of 4096 and more fill most CUs: gate+up at 17 / 32 /
+//   64 rows 30.9 / 31.5 / 41.3 and 28.4 / 29.6 / 41.1 (64 rows with its weights in the
+//   last-level cache 43 and 36), 2 x 11008x4096 at 32 rows 31.3 and 29.2; nor with f16
+//   outputs and a k up to 1024: 2 x 4864x896 at 24 to 64 rows 9 to 10 % the other way; nor where
+//   a k under 1024 is split there and not here, a launch less: 1536x576 at 17 rows 10.3 and 10.7 in
+//   a graph, 2064x848 at 22 rows 14.7 and 11.1 from eager calls.
+//   Above, the estimate decides, with 6 % in hand for its error (f16 outputs 0 to 8 %), and where it
+//   was wrong too often (f32 outputs at a k under 1024 or up to 128 rows), these lines do:
+//   Exact, from a k of 4096 and enough products per launch for the larger item costs: q/k/v at
+//   128 rows 31.3 and 30.3, o at 192 rows 28.5 and 27.1, 8192x8192 at 100 rows 44.2 and 42.3, but
+//   o at 128 rows 22.7 and 23.2 and, its blocks not full, down at 100 rows 37.1 and 38.1; shorter k
+//   from 256 rows: 2 x 4096x2048 at 256 rows 30.0 and 31.5, at 768 rows 80.8 and 69.6.
+//   fp16-weight mode, k of 8192 and more: down at 512 rows 81.7 and 73.5, 8192x8192 at 384 rows 5 %
+//   the other way.
+//   1MAD: half the products in the streaming kernels' exact mode, a cheaper decode in both. Exact,
+//   o at 24 / 64 rows 14.7 / 17.7 and 14.0 / 17.0, gate+up at 64 rows 51.7 and 38.8, 2048x2048 at 24 /
+//   100 rows 12.0 / 14.2 and 12.4 / 15.1; fp16-weight mode, down at 1024 rows 174 and 138, but 2 x
+//   4096x1024 at 512 rows 28.0 and 32.9.
+bool streams(const trellis_desc* const* W, int count, int batch, bool f16, bool y_f16, const BgPlan& sh,
+             const BgPlan& st) {
   int maxt = 0;
-  for (int i = 0; i < count; ++i) maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
-  const bool longk = maxt >= 512;
-  const bool shortk = maxt <= 64;
-  if (f16) return batch <= 64 || shortk || (batch <= 512 && !longk);
-  return W[0]->codebook != TRELLIS_CB_1MAD && (batch <= 64 ? longk : batch <= 128 && shortk);
+  long long products = 0;
+  int blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    maxt = W[i]->k_in / 16 > maxt ? W[i]->k_in / 16 : maxt;
+    products += static_cast<long long>(batch) * W[i]->n_out * W[i]->k_in;
+    blocks += (W[i]->n_out + 127) / 128;
+  }
+  if (W[0]->codebook == TRELLIS_CB_1MAD && (!f16 || maxt > 64))
+    return products >= (y_f16 ? 300000000LL : 600000000LL);
+  if (batch <= 64)
+    return !f16 && ((count > 1 && maxt >= 256 && st.smax == 1) ||
+                    (y_f16 && maxt <= 64) || (maxt < 64 && st.smax == 1 && sh.smax > 1));
+  if (f16 && batch > 384 && maxt >= 512) return true;
+  const int hand = !y_f16 ? 106 : f16 ? 103 : batch > 128 ? 100 : 108;
+  if ((y_f16 || (batch > 128 && maxt >= 64)) &&
+      call_ns(st, f16, y_f16) * hand < call_ns(sh, f16, y_f16) * 100)
+    return true;
+  if (f16) return false;
+  if (maxt >= 256 && products >= 2500000000LL && (batch >= 112 || blocks >= 48)) return true;
+  return batch > 256 && maxt >= 112 && products >= 1000000000LL;
 }
 
-// Column-block width in 16-column units: 1 up to 16 rows, 2 up to 32; above, the width that
-// the model above finds cheapest for the group, of 32 and 64 columns up to 64 rows (at 64
-// rows the 8B o launch takes 17.5 us in 32-column blocks and 19.7 in 64-column ones, gate+up
-// 53.7 and 40.8), else of 64, 128 and 256 (gate+up at 512 rows 246, 205 and 222 us, at 1024
-// rows 472, 395 and 365; o at 256 rows 33.0, 33.5 and 39.5).
-int bgemm_nc(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn) {
-  if (kn.bgemm_nc) return kn.bgemm_nc;
-  if (batch <= 16) return 1;
-  if (batch <= 32) return 2;
-  int best = 0;
-  long long best_cost = 0;
-  for (int nc = batch <= 64 ? 2 : 4; nc <= (batch <= 64 ? 4 : 16); nc *= 2) {
-    long long c;
-    bgemm_kr_cost(W, count, batch, nc, f16, false, true, kn, &c);
-    if (best == 0 || c < best_cost) {
-      best = nc;
-      best_cost = c;
-    }
+// Which kernels a plan may take: the rule's choice, or one of them for sizing a workspace.
+enum class Batched { rule, shared, streaming };
+
+BgPlan plan_batched(const trellis_desc* const* W, int count, int batch, bool f16, bool y_f16, Batched which,
+                    bool split, const Knobs& kn) {
+  if (kn.bgemm_nc) which = kn.bgemm_nc == 1 ? Batched::shared : Batched::streaming;
+  else if (batch <= 16) which = Batched::shared;
+  if (which == Batched::rule) {
+    // chosen on the plans with a split of k, whether or not this one may split
+    const BgPlan sh = plan_shared(W, count, batch, f16, true, kn);
+    const BgPlan st = plan_streaming(W, count, batch, f16, true, kn);
+    which = streams(W, count, batch, f16, y_f16, sh, st) ? Batched::streaming : Batched::shared;
+    if (split) return which == Batched::shared ? sh : st;
   }
-  return best;
+  return which == Batched::shared ? plan_shared(W, count, batch, f16, split, kn)
+                                  : plan_streaming(W, count, batch, f16, split, kn);
 }
 
 // The decode-GEMV for batch 1 to 4, and for 5 to 16 when its items at the longest k-range
@@ -339,16 +411,16 @@ size_t xf_bytes(bool frag, int batch, int k) {
 }
 
 // `split` off: the batched path's k-ranges are whole (no partial sums in the workspace).
-GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f16, const Knobs& kn,
-                     bool split_k = true) {
+GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f16, bool y_f16, const Knobs& kn,
+                     bool split_k = true, Batched which = Batched::rule) {
   GroupPlan p;
   p.gemv = use_gemv(W, count, batch, kn);
   p.nb = batch;
-  p.shared = bgemm_shared(W, count, batch, f16, kn);
-  p.nc = !p.shared ? bgemm_nc(W, count, batch, f16, kn)
-                   : kn.bgemm_nc == 1 || batch <= 16 ? 1 : batch <= 32 ? 2 : batch <= 64 || !f16 ? 4 : 8;
+  const BgPlan b = p.gemv ? BgPlan() : plan_batched(W, count, batch, f16, y_f16, which, split_k, kn);
+  p.shared = b.shared;
+  p.nc = b.nc;
   p.ncb = p.gemv ? 1 : (batch + 16 * p.nc - 1) / (16 * p.nc);
-  p.kr = p.gemv ? gemv_kr(W, count, batch, kn) : bgemm_kr(W, count, batch, p.nc, f16, p.shared, split_k, kn);
+  p.kr = p.gemv ? gemv_kr(W, count, batch, kn) : b.kr;
   // tiles per decode-GEMV stage: 16, or 8 for short k-ranges and for launches that split k
   // (a workgroup's first stage lands sooner: the 8B block's q/k/v and down launches
   // 0.2-0.7 us faster each at batch 1 to 8)
@@ -363,7 +435,6 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
   // kernel's stages are 8 tiles; the plan says so too
   if (p.gemv && gemv_nb(batch) == 16) p.kc = 8;
   p.total = 0;
-  p.folds = 0;
   // Workspace: a header of counters whose layout depends only on the members' shapes (one
   // split-K ticket per 128-row block of every member); every call leaves them at zero.
   // Plans for other batch sizes reuse the same workspace, so their data (partial sums,
@@ -381,7 +452,6 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
   for (int i = 0; i < count; ++i) {
     p.S[i] = (W[i]->k_in / 16 + p.kr - 1) / p.kr;
     p.total += p.n_ob[i] * p.ncb * p.S[i];
-    p.folds += p.nb * ((W[i]->k_in + 127) / 128);
     p.off_part[i] = p.ws;
     if (p.S[i] > 1)
       p.ws += align256(static_cast<size_t>(p.n_ob[i]) * p.ncb * p.S[i] * part_cols * 128 *
@@ -395,18 +465,20 @@ GroupPlan group_plan(const trellis_desc* const* W, int count, int batch, bool f1
 // Workspace bytes that cover every call of up to `batch` rows, in either MFMA mode (their
 // k-ranges, hence partial buffers, may differ). A smaller batch can need more: fewer column
 // blocks leave CUs idle that a split of k then fills (4096 x 4096 at K=3: 25.2 MB at 512 rows,
-// 8.4 MB at 513). A plan's choices change with the batch only at 1, 2, 4, 8, 16, 32 and 64 rows
+// 8.4 MB at 513). A kernel's plan changes with the batch only at 1, 2, 4, 8, 16, 32 and 64 rows
 // and where another column block starts, 64 columns or more apart above 64 rows; up to the next
-// such end it grows with the rows, so only the ends and `batch` itself are planned.
+// such end it grows with the rows, so only the ends and `batch` itself are planned, with either
+// batched kernel.
 size_t covering_ws(const trellis_desc* const* W, int count, int batch, const Knobs& kn) {
   const int step = kn.bgemm_nc == 1 ? 16 : kn.bgemm_nc == 2 ? 32 : 64;
   size_t most = 0;
   for (int b = 1;;) {
     const int at = b < batch ? b : batch;
-    for (const bool f16 : {false, true}) {
-      const size_t ws = group_plan(W, count, at, f16, kn).ws;
-      most = ws > most ? ws : most;
-    }
+    for (const bool f16 : {false, true})
+      for (const Batched which : {Batched::shared, Batched::streaming}) {
+        const size_t ws = group_plan(W, count, at, f16, false, kn, true, which).ws;
+        most = ws > most ? ws : most;
+      }
     if (at == batch) return most;
     b = b < step ? 2 * b : b > batch - step ? batch : b + step;
   }
@@ -736,11 +808,12 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
     if (static_cast<int64_t>(batch) * (batch > 1 ? ldx[i] : W[i]->k_in) * xes >= (int64_t(1) << 31))
       return TRELLIS_ERR_SHAPE;
   }
-  GroupPlan p = group_plan(W, count, batch, f16, kn);
+  const bool y_f16 = y_dtype == TRELLIS_F16;
+  GroupPlan p = group_plan(W, count, batch, f16, y_f16, kn);
   if (noalloc) {
     // a batched plan whose partial sums do not fit the scratch goes without a split of k:
     // what is left is the folded activations
-    if (p.ws > NOALLOC_SCRATCH_BYTES && !p.gemv) p = group_plan(W, count, batch, f16, kn, false);
+    if (p.ws > NOALLOC_SCRATCH_BYTES && !p.gemv) p = group_plan(W, count, batch, f16, y_f16, kn, false);
     if (p.ws > NOALLOC_SCRATCH_BYTES) return TRELLIS_ERR_SCRATCH;
     v = scratch_ptr(static_cast<hipStream_t>(stream), &workspace);
     if (v) return v;
@@ -756,7 +829,7 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
   g.total = p.total;
   g.nwords = W[0]->nwords;
   g.x_f16 = x_dtype == TRELLIS_F16;
-  g.y_f16 = y_dtype == TRELLIS_F16;
+  g.y_f16 = y_f16;
   g.kr = p.kr;
   g.mma_f16 = f16;
   int item0 = 0;
@@ -801,9 +874,9 @@ int packed_linear_group(const trellis_desc* const* W, int count, const void* con
   }
   if (kn.plan_log)
     std::fprintf(stderr, "trellis plan: batch=%d members=%d mode=%s kr=%d kc=%d nc=%d ncb=%d "
-                         "items=%d S0=%d ws=%zu\n",
+                         "items=%d S0=%d ws=%zu shared=%d\n",
                  batch, count, p.gemv ? "gemv" : f16 ? "bgemm-f16" : "bgemm", p.kr, p.kc, p.nc,
-                 p.ncb, p.total, p.S[0], p.ws);
+                 p.ncb, p.total, p.S[0], p.ws, static_cast<int>(p.shared));
   if (noalloc && p.gemv) {
     // only the decode-GEMV's split-K tickets must start at zero (the batched path writes
     // its folded activations and partial sums before reading them)
