@@ -20,7 +20,7 @@ n*k*K/8). The JSON line also carries us/layer, the dominant launch's HBM rooflin
 duration from HIP events on the launch stream), the same block at batch 16 and 64 and at a
 512-token prefill with their fp16 MFMA rooflines (algorithmic 2*B*n*k flops), and a CPU baseline: this repo's torch-CPU
 restatement of the reference decode+restore+matmul (oracle/torch_cpu.py) on a bounded
-sample, per configuration and layer. The bit-rate sweep (configs[4]: K=2,3,4 x V=1,2 on
+sample, per configuration and layer. The bit-rate sweep (K=2,3,4 x V=1,2 on
 the 8B gate/up/down shapes, at batch 1 and at a 512-token prefill) runs by default
 (--no-sweep skips it), each point with its own roofline.
 
@@ -270,14 +270,14 @@ def run_block(te, torch, dev, layers, groups, B, K, V, steps, warmup, min_bytes=
 # the benchmark per layer (the 8B block's v, o and up have the shapes of k, q and gate) and
 # one point of the bit-rate sweep.
 CPU_LAYERS = [
-    ("configs[0] SmolLM2-135M", "up_proj", 1536, 576, 3, "3inst"),
-    ("configs[1] Qwen3-1.7B MLP", "gate/up", 6144, 2048, 3, "mcg"),
-    ("configs[1] Qwen3-1.7B MLP", "down", 2048, 6144, 3, "mcg"),
-    ("configs[2] Qwen3-8B block", "q/o", 4096, 4096, 3, "mcg"),
-    ("configs[2] Qwen3-8B block", "k/v", 1024, 4096, 3, "mcg"),
-    ("configs[2] Qwen3-8B block", "gate/up", 12288, 4096, 3, "mcg"),
-    ("configs[2] Qwen3-8B block", "down", 4096, 12288, 3, "mcg"),
-    ("configs[4] sweep K=4", "gate/up", 12288, 4096, 4, "mcg"),
+    ("SmolLM2-135M", "up_proj", 1536, 576, 3, "3inst"),
+    ("Qwen3-1.7B MLP", "gate/up", 6144, 2048, 3, "mcg"),
+    ("Qwen3-1.7B MLP", "down", 2048, 6144, 3, "mcg"),
+    ("Qwen3-8B block", "q/o", 4096, 4096, 3, "mcg"),
+    ("Qwen3-8B block", "k/v", 1024, 4096, 3, "mcg"),
+    ("Qwen3-8B block", "gate/up", 12288, 4096, 3, "mcg"),
+    ("Qwen3-8B block", "down", 4096, 12288, 3, "mcg"),
+    ("sweep K=4", "gate/up", 12288, 4096, 4, "mcg"),
 ]
 # how many times each 8B shape occurs in the block (q, k, v, o, gate, up, down)
 BLOCK_MULT = {"q/o": 2, "k/v": 2, "gate/up": 2, "down": 1}
@@ -325,7 +325,7 @@ def cpu_baseline(budget_s: float = 30.0):
                           "matmul_only_ms": round(b * 1e3, 3),
                           "packed_GBps": round(pb / a / 1e9, 4)})
         log(f"[bench] cpu {cfg} {layer} {n}x{k} K={K}: {a * 1e3:.1f} ms (matmul {b * 1e3:.2f} ms)")
-        if cfg.startswith("configs[2]"):
+        if cfg.startswith("Qwen3-8B"):
             block_s += BLOCK_MULT[layer] * a
     total_s = time.perf_counter() - t_start
     block_bytes = sum(n * k * 3 // 8 for _, n, k in LAYERS)
@@ -473,7 +473,6 @@ def batched_figure(te, torch, dev, bs, K, V, args, samples=None):
     dom_fl = 2 * bs * 2 * 12288 * 4096
     dom_tf = dom_fl / (grp[DOMINANT] * 1e-6) / 1e12
     # the planner's width for gate+up (above 64 columns: 128 here, by its cost model)
-    nc = 1 if bs <= 16 else 2 if bs <= 32 else 4 if bs <= 64 else 8
     out = {"us_per_block": round(sec * 1e6, 2),
            "us_per_block_one_graph_per_block": round(ge["sec"] * 1e6, 2),
            "blocks_per_graph": copies,
@@ -483,7 +482,7 @@ def batched_figure(te, torch, dev, bs, K, V, args, samples=None):
            "roofline": {"bound": "mfma", "achieved": round(dom_tf, 2),
                         "peak": MFMA_FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
                         "frac": round(dom_tf / MFMA_FP16_PEAK_TFLOPS, 4),
-                        "kernel": f"bgemm_kernel<K={K},MCG,V={V},NC={nc}> (+xfold, bfold) "
+                        "kernel": f"batched kernel (csrc/bgemm.h) K={K},MCG,V={V} (+xfold, bfold) "
                                   f"on gate+up at batch {bs}",
                         "avg_launch_us": grp[DOMINANT],
                         "algorithmic_flops_per_launch": dom_fl}}
@@ -693,7 +692,7 @@ def main():
                                        "known size)",
                      "kernel": f"gemv_kernel<K={K},MCG,V={V}> on the gate+up group "
                                "(2 x 12288x4096, one launch)" if B == 1 else
-                               f"bgemm_kernel<K={K},MCG,V={V}> on the gate+up group",
+                               f"batched kernel (csrc/bgemm.h) K={K},MCG,V={V} on the gate+up group",
                      "avg_launch_us": round(dom_us, 3),
                      "algorithmic_bytes_per_launch": dom_bytes},
     }
