@@ -472,7 +472,6 @@ def batched_figure(te, torch, dev, bs, K, V, args, samples=None):
     fl = block_flops(LAYERS, bs)
     dom_fl = 2 * bs * 2 * 12288 * 4096
     dom_tf = dom_fl / (grp[DOMINANT] * 1e-6) / 1e12
-    # the planner's width for gate+up (above 64 columns: 128 here, by its cost model)
     out = {"us_per_block": round(sec * 1e6, 2),
            "us_per_block_one_graph_per_block": round(ge["sec"] * 1e6, 2),
            "blocks_per_graph": copies,
