@@ -68,7 +68,8 @@ def test_shared_activation_kernel(te, gpu_device, monkeypatch, capfd, n, k, K, c
 
 
 @pytest.mark.parametrize("kr", ["0", "24"])      # the planner's, and one that splits the longer k
-@pytest.mark.parametrize("n,k,K,cb,V,batch", [(12304, 336, 3, "mcg", 1, 129), (4112, 528, 2, "3inst", 2, 760)])
+@pytest.mark.parametrize("n,k,K,cb,V,batch", [(12304, 336, 3, "mcg", 1, 129), (4112, 528, 2, "3inst", 2, 760),
+                                              (12304, 336, 4, "1mad", 1, 129)])
 def test_shared_exact_128_columns(te, gpu_device, monkeypatch, capfd, kr, n, k, K, cb, V, batch):
     """Its 12-wave instantiation (exact mode, 128 columns, steps of 6 tile columns), single and in
     a group, with k-ranges that end inside a step and ragged last column blocks."""

@@ -236,31 +236,26 @@ BgPlan bgemm_plan(const trellis_desc* const* W, int count, int batch, int nc, bo
   const int forced = kn.bgemm_kr;
   const bool force = split && forced >= kt && forced % kt == 0;
   BgPlan best;
-  // members of one k: of the k-ranges that cut it into S slices the shortest is the cheapest, so
-  // those of S = 16 .. 1 are looked at (a call's host time pays for the search)
-  bool one_k = true;
-  for (int i = 1; i < count; ++i) one_k = one_k && W[i]->k_in == W[0]->k_in;
-  const auto shortest = [&](int S) { return ((maxt + S - 1) / S + kt - 1) / kt * kt; };
-  int S1 = 16;
-  for (int kr = !split ? cap : force ? (forced < cap ? forced : cap) : one_k ? shortest(S1) : kt; kr <= cap;) {
+  // of the k-ranges that cut the members into the same slices the shortest is the cheapest, so from
+  // 16 slices of the longest k only those are looked at where a member's count falls (a call's host
+  // time pays for the search)
+  const auto shortest = [kt](int t, int S) { return ((t + S - 1) / S + kt - 1) / kt * kt; };
+  for (int kr = !split ? cap : force ? (forced < cap ? forced : cap) : shortest(maxt, 16); kr <= cap;) {
     long long items = 0, part_bytes = 0;
-    int smax = 1;
+    int smax = 1, next = cap + 1;
     for (int i = 0; i < count; ++i) {
-      const int S = (W[i]->k_in / 16 + kr - 1) / kr;
+      const int t = W[i]->k_in / 16, S = (t + kr - 1) / kr;
       const long long n_ob = (W[i]->n_out + 127) / 128;
       items += n_ob * ncb * S;
       smax = S > smax ? S : smax;
+      if (S > 1 && shortest(t, S - 1) < next) next = shortest(t, S - 1);
       if (S > 1) part_bytes += static_cast<long long>(S) * n_ob * ncb * 128 * 16 * nc * 4;
     }
     const long long rounds = (items + cus - 1) / cus;
     const long long c = rounds * (2LL * kr * bc.tile + bc.item) +
                         (smax > 1 ? bc.fold + part_bytes / bc.bytes : 0);
-    if ((smax <= 16 || force) && (best.cost < 0 || c < best.cost))
-      best = {shared, nc, kr, smax, c, rounds, part_bytes};
-    if (force || kr == cap) break;
-    int next = kr + kt;
-    if (one_k)
-      while (S1 > 1 && (next = shortest(--S1)) == kr) {}
+    if (best.cost < 0 || c < best.cost) best = {shared, nc, kr, smax, c, rounds, part_bytes};
+    if (force) break;
     kr = next;
   }
   return best;
@@ -347,11 +342,11 @@ bool streams(const trellis_desc* const* W, int count, int batch, bool f16, bool 
     products += static_cast<long long>(batch) * W[i]->n_out * W[i]->k_in;
     blocks += (W[i]->n_out + 127) / 128;
   }
+  const bool launch_less = !f16 && batch <= 64 && maxt < 64 && st.smax == 1 && sh.smax > 1;
   if (W[0]->codebook == TRELLIS_CB_1MAD && (!f16 || maxt > 64))
-    return products >= (y_f16 ? 300000000LL : 600000000LL);
+    return products >= (y_f16 ? 300000000LL : 600000000LL) || launch_less;
   if (batch <= 64)
-    return !f16 && ((count > 1 && maxt >= 256 && st.smax == 1) ||
-                    (y_f16 && maxt <= 64) || (maxt < 64 && st.smax == 1 && sh.smax > 1));
+    return !f16 && ((count > 1 && maxt >= 256 && st.smax == 1) || (y_f16 && maxt <= 64) || launch_less);
   if (f16 && batch > 384 && maxt >= 512) return true;
   const int hand = !y_f16 ? 106 : f16 ? 103 : batch > 128 ? 100 : 108;
   if ((y_f16 || (batch > 128 && maxt >= 64)) &&
