@@ -105,7 +105,7 @@ __device__ __forceinline__ void st_wt(_Float16* p, _Float16 v) {
 // need two wait states, one more than gfx90a, between a store of more than 8 bytes and a VALU
 // write of its data registers, and the compiler's hazard pass does not look inside inline
 // assembly. The registers are free after the store, so the next address computed may take them:
-// with one wait state two of its 16 bytes' words could leave as the halves of that address. A
+// with one wait state two of the four words stored could be the halves of that address. A
 // buffer store, which the pass does see, would bound the rows' stride by its 32-bit offsets.)
 __device__ __forceinline__ void st_wt16(void* p, u32x4_t v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
